@@ -20,6 +20,7 @@
 
 #include "host_ops.hpp"
 #include "dg_batch.hpp"
+#include "transfer.hpp"
 
 namespace {
 
@@ -104,6 +105,7 @@ void free_batch(Batch* b) {
     (void)hipFree(b->margs);
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
     if (b->stream) (void)hipStreamDestroy(b->stream);
+    staging_release();
 }
 
 template <int M, typename Real>
@@ -390,6 +392,7 @@ int nemo_gpu_batch_create(const nemo_gpu_config* cfg, int32_t nruns, const int32
     for (int r = 0; r < nruns; ++r)
         if (n_poly[r] < 2 || n_poly[r] > 4 || nelem[r] <= 0) return fail(NEMO_ERR_ARG, "run with invalid n_poly or size");
     Batch* b = new Batch();
+    staging_retain();
     b->cfg = *cfg;
     b->nruns = nruns;
     b->rk = make_rk();
@@ -507,13 +510,10 @@ int nemo_gpu_batch_upload(void* handle, int32_t run, const int32_t* nbr, const d
     HIP_TRY(hipStreamSynchronize(b->stream));
     HIP_TRY(hipMemcpy(gr.nbr + off * 6, n.data(), n.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(gr.delta + off * 3, delta, size_t(ne) * 3 * sizeof(double), hipMemcpyHostToDevice));
-    std::vector<double> col(size_t(ne) * M3);
-    for (int v = 0; v < 5; ++v) {
-        for (long long e = 0; e < ne; ++e)
-            std::memcpy(&col[size_t(e) * M3], &u[(size_t(e) * 5 + v) * M3], M3 * sizeof(double));
-        HIP_TRY(hipMemcpy(gr.u[gr.cur] + (size_t(v) * gr.nelem + off) * M3, col.data(), col.size() * sizeof(double),
-                          hipMemcpyHostToDevice));
-    }
+    // the run's share of the idle ping-pong buffer takes the host layout
+    HIP_TRY(state_to_device(b->stream, u, gr.u[gr.cur ^ 1] + size_t(5) * off * M3, gr.u[gr.cur], gr.nelem, off, ne, 5,
+                            M3));
+    HIP_TRY(hipStreamSynchronize(b->stream));
     return NEMO_OK;
 }
 
@@ -523,14 +523,8 @@ int nemo_gpu_batch_download(void* handle, int32_t run, double* u) {
     Group& gr = b->g[b->run_group[run]];
     const long long ne = b->run_nelem[run], off = b->run_off[run];
     const int M3 = gr.M * gr.M * gr.M;
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    std::vector<double> col(size_t(ne) * M3);
-    for (int v = 0; v < 5; ++v) {
-        HIP_TRY(hipMemcpy(col.data(), gr.u[gr.cur] + (size_t(v) * gr.nelem + off) * M3, col.size() * sizeof(double),
-                          hipMemcpyDeviceToHost));
-        for (long long e = 0; e < ne; ++e)
-            std::memcpy(&u[(size_t(e) * 5 + v) * M3], &col[size_t(e) * M3], M3 * sizeof(double));
-    }
+    HIP_TRY(state_to_host(b->stream, gr.u[gr.cur], gr.nelem, off, ne, 5, M3, gr.u[gr.cur ^ 1] + size_t(5) * off * M3,
+                          u));
     return NEMO_OK;
 }
 

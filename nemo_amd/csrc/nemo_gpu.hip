@@ -18,6 +18,7 @@
 #include "../../include/nemo_gpu.h"
 #include "host_ops.hpp"
 #include "solver.hpp"
+#include "transfer.hpp"
 #include "dg_mortar.hpp"
 #include "dg_analyze.hpp"
 
@@ -165,22 +166,6 @@ int check_ready(Solver* s) {
     if (!s->have_mesh) return fail(NEMO_ERR_NOT_READY, "mesh not uploaded");
     if (!s->have_state) return fail(NEMO_ERR_NOT_READY, "state not uploaded");
     return NEMO_OK;
-}
-
-// host layout u[e][v][n]  <->  device layout u[v][e][n]
-void to_device_layout(const Solver& s, const double* host, std::vector<double>& dev) {
-    dev.resize(s.state_doubles());
-    const size_t M3 = s.M3, E = s.nelem;
-    for (size_t e = 0; e < E; ++e)
-        for (int v = 0; v < s.V; ++v)
-            std::memcpy(&dev[(v * E + e) * M3], &host[(e * s.V + v) * M3], M3 * sizeof(double));
-}
-
-void to_host_layout(const Solver& s, const std::vector<double>& dev, double* host) {
-    const size_t M3 = s.M3, E = s.nelem;
-    for (size_t e = 0; e < E; ++e)
-        for (int v = 0; v < s.V; ++v)
-            std::memcpy(&host[(e * s.V + v) * M3], &dev[(v * E + e) * M3], M3 * sizeof(double));
 }
 
 int status_check(Solver* s) {
@@ -423,6 +408,7 @@ int nemo_gpu_create(const nemo_gpu_config* cfg, void** handle) {
         delete s;
         return fail(NEMO_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
     }
+    staging_retain();
     if (hipMalloc(&s->dt_dev, 8 * sizeof(double)) != hipSuccess ||
         hipMalloc(&s->mlp_p, nemo::MLP_NP * sizeof(float)) != hipSuccess ||
         hipMalloc(&s->mlp_inf, nemo::MLP_NP * sizeof(float)) != hipSuccess ||
@@ -473,6 +459,7 @@ int nemo_gpu_destroy(void* handle) {
         (void)hipEventDestroy(p.second);
     }
     (void)hipStreamDestroy(s->stream);
+    staging_release();
     delete s;
     return NEMO_OK;
 }
@@ -564,10 +551,9 @@ int nemo_gpu_upload_state(void* handle, const double* u) {
     Solver* s = static_cast<Solver*>(handle);
     if (!s || !u) return fail(NEMO_ERR_ARG, "null argument");
     if (!s->have_mesh) return fail(NEMO_ERR_NOT_READY, "mesh not uploaded");
-    std::vector<double> dev;
-    to_device_layout(*s, u, dev);
     const size_t bytes = s->state_doubles() * sizeof(double);
-    HIP_TRY(hipMemcpyAsync(s->u[s->cur], dev.data(), bytes, hipMemcpyHostToDevice, s->stream));
+    // the idle ping-pong buffer takes the host layout
+    HIP_TRY(state_to_device(s->stream, u, s->u[s->cur ^ 1], s->u[s->cur], s->nelem, 0, s->nelem, s->V, s->M3));
     HIP_TRY(hipMemsetAsync(s->r0, 0, bytes, s->stream));
     HIP_TRY(hipMemsetAsync(s->r1, 0, bytes, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
@@ -579,10 +565,7 @@ int nemo_gpu_download_state(void* handle, double* u) {
     Solver* s = static_cast<Solver*>(handle);
     if (int rc = check_ready(s)) return rc;
     if (!u) return fail(NEMO_ERR_ARG, "null argument");
-    std::vector<double> dev(s->state_doubles());
-    HIP_TRY(hipMemcpyAsync(dev.data(), s->u[s->cur], dev.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    to_host_layout(*s, dev, u);
+    HIP_TRY(state_to_host(s->stream, s->u[s->cur], s->nelem, 0, s->nelem, s->V, s->M3, s->u[s->cur ^ 1], u));
     return NEMO_OK;
 }
 
@@ -591,10 +574,7 @@ int nemo_gpu_rhs(void* handle, double* rhs) {
     if (int rc = check_ready(s)) return rc;
     if (!rhs) return fail(NEMO_ERR_ARG, "null argument");
     if (int rc = launch_stage(*s, 1, 0.0, nullptr, s->rhs, nullptr)) return rc;
-    std::vector<double> dev(s->state_doubles());
-    HIP_TRY(hipMemcpyAsync(dev.data(), s->rhs, dev.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    to_host_layout(*s, dev, rhs);
+    HIP_TRY(state_to_host(s->stream, s->rhs, s->nelem, 0, s->nelem, s->V, s->M3, s->u[s->cur ^ 1], rhs));
     return NEMO_OK;
 }
 
