@@ -835,9 +835,11 @@ int nemo_gpu_mlp_forward(void* handle, int64_t n, const float* features, float* 
     }
     hipError_t e = hipMemcpyAsync(df, features, size_t(n) * 4 * sizeof(float), hipMemcpyHostToDevice, s->stream);
     if (e == hipSuccess) {
-        const long long groups = (n + 3) / 4;
-        hipLaunchKernelGGL(nemo::mlp_forward_kernel, dim3(unsigned(groups < 65536 ? groups : 65536)), dim3(64), 0,
-                           s->stream, s->mlp_inf, (long long)n, df, dy);
+        // up to four workgroups per CU, so that each loads the weights once
+        // for several tiles
+        const long long tiles = (n + nemo::MLP_TILE - 1) / nemo::MLP_TILE;
+        hipLaunchKernelGGL(nemo::mlp_forward_kernel, dim3(unsigned(tiles < 1024 ? tiles : 1024)), dim3(nemo::MLP_NT),
+                           0, s->stream, s->mlp_p, (long long)n, df, dy);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(y, dy, size_t(n) * sizeof(float), hipMemcpyDeviceToHost, s->stream);
@@ -850,15 +852,22 @@ int nemo_gpu_mlp_forward(void* handle, int64_t n, const float* features, float* 
 
 namespace {
 
+// Gradient partials of a minibatch of n samples: one per tile, at most one
+// workgroup per CU.
+int mlp_parts(long long n) {
+    const long long tiles = (n + nemo::MLP_TILE - 1) / nemo::MLP_TILE;
+    return int(tiles < nemo::MLP_PARTS ? tiles : nemo::MLP_PARTS);
+}
+
 // One minibatch: partial gradients per block, then the ordered reduction
 // (and an Adam step when lr > 0).
 int mlp_batch(Solver* s, const float* df, const float* dt, const long long* didx, long long off, int B, float* part,
               float* part_loss, float* dgrad, float* dloss, int nparts, float lr, long long t) {
-    hipLaunchKernelGGL(nemo::mlp_grad_kernel, dim3(nparts), dim3(64), 0, s->stream, s->mlp_p, df, dt, didx, off, B,
+    hipLaunchKernelGGL(nemo::mlp_grad_kernel, dim3(nparts), dim3(nemo::MLP_NT), 0, s->stream, s->mlp_p, df, dt, didx, off, B,
                        part, part_loss);
     HIP_TRY(hipGetLastError());
     const float c1 = float(1.0 - std::pow(0.9, double(t))), c2 = float(1.0 - std::pow(0.999, double(t)));
-    hipLaunchKernelGGL(nemo::mlp_reduce_kernel, dim3((nemo::MLP_NP + 255) / 256), dim3(256), 0, s->stream, part,
+    hipLaunchKernelGGL(nemo::mlp_reduce_kernel, dim3((nemo::MLP_NP + 63) / 64), dim3(64 * nemo::MLP_RW), 0, s->stream, part,
                        nparts, part_loss, dgrad, dloss, s->mlp_p, s->mlp_m, s->mlp_v, lr > 0.0f ? 1 : 0, lr, c1, c2);
     HIP_TRY(hipGetLastError());
     return NEMO_OK;
@@ -875,7 +884,7 @@ int nemo_gpu_mlp_grad(void* handle, int64_t n, const float* features, const floa
                       float* grad) {
     Solver* s = static_cast<Solver*>(handle);
     if (!s || !features || !target || n <= 0 || n > (1 << 30)) return fail(NEMO_ERR_ARG, "invalid arguments");
-    const int nparts = int(n < 128 ? n : 128);
+    const int nparts = mlp_parts(n);
     DevBuf f, t, part, pl, g, l;
     HIP_TRY(hipMalloc(&f.p, size_t(n) * 4 * sizeof(float)));
     HIP_TRY(hipMalloc(&t.p, size_t(n) * sizeof(float)));
@@ -902,7 +911,7 @@ int nemo_gpu_mlp_train(void* handle, int64_t n, const float* features, const flo
     if (!s || !features || !target || n <= 0 || epochs <= 0 || batch <= 0 || !(lr > 0.0f))
         return fail(NEMO_ERR_ARG, "invalid arguments");
     if (!s->mlp_ready) return fail(NEMO_ERR_NOT_READY, "set initial parameters first (nemo_gpu_mlp_set_params)");
-    const int nparts = batch < 128 ? batch : 128;
+    const int nparts = mlp_parts(batch);
     DevBuf f, t, idx, part, pl, l;
     HIP_TRY(hipMalloc(&f.p, size_t(n) * 4 * sizeof(float)));
     HIP_TRY(hipMalloc(&t.p, size_t(n) * sizeof(float)));
