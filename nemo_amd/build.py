@@ -29,7 +29,8 @@ def _run(cmd, cwd=ROOT):
     return out
 
 
-HIP_SOURCES = ["nemo_gpu.hip", "stage_m3.hip", "stage_m4.hip", "stage_m5.hip", "batch.hip", "transfer.hip"]
+HIP_SOURCES = ["nemo_gpu.hip", "stage_m3.hip", "stage_m4.hip", "stage_m5.hip",
+               "wide_m3.hip", "wide_m4.hip", "wide_m5.hip", "batch.hip", "transfer.hip"]
 
 
 def build_hip(verbose: bool = False) -> str:

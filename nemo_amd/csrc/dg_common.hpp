@@ -162,6 +162,20 @@ __device__ __forceinline__ long long xcd_block(long long nblocks) {
     return (bid & 7) * per + (bid >> 3);
 }
 
+// Orders a wavefront's LDS accesses among its lanes: a barrier where the
+// workgroup is that one wavefront; with SHARED (other wavefronts of the
+// workgroup do something else) a fence, since the LDS accesses of one
+// wavefront execute in order.
+template <bool SHARED>
+__device__ __forceinline__ void wave_sync() {
+    if constexpr (SHARED) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
 // A compile-time flag passed as an argument (selects a variant of a pass).
 template <bool B>
 struct BoolConst {

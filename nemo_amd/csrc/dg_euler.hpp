@@ -88,19 +88,17 @@ __device__ __forceinline__ void load_face_nodes(const StageArgs<M, Real>& a, lon
     }
 }
 
-// Surface term of direction D: the two face Riemann problems of the thread's
-// line and their lifting to the end nodes, +jac f*_- / w_0 and
-// -jac f*_+ / w_{M-1}.  With LGL subcells the DG and FV surface terms are the
-// same, so the term does not depend on the blending factor and is added to
-// the accumulators before the volume passes (pass D = 0 initialises them).
-template <int D, int M, int BE, int SURF, typename Real, typename TU>
-__device__ __forceinline__ void surface_pass(const StageArgs<M, Real>& a, long long e0, const TU (*s_u)[BE * M * M * M],
-                                             Real (*s_acc)[BE * M * M * M], const double* s_p64, const ElemGeom& geo,
-                                             const FaceNodes& fn) {
+// The two face Riemann fluxes of line `tid` in direction D from the nodes um
+// and up across its ends, and jac = 2 / dx.  In the FP32 operator with INBLK
+// a neighbour inside the block is read from LDS (load_face_nodes).
+template <int D, int M, int BE, int SURF, bool INBLK, typename Real, typename TU>
+__device__ __forceinline__ void surface_fluxes(const StageArgs<M, Real>& a, int tid, long long e0,
+                                               const TU (*s_u)[BE * M * M * M], const double* s_p64,
+                                               const ElemGeom& geo, const double (&um)[5], const double (&up)[5],
+                                               Real (&fm)[5], Real (&fp)[5], Real& jac) {
     using Sh = StageShape<M, BE>;
     constexpr int M2 = Sh::M2, M3 = Sh::M3;
     constexpr bool F32 = sizeof(Real) == 4;
-    const int tid = threadIdx.x;
     const int el = tid / M2;
     const int line = tid - el * M2;
     const int ta = line % M, tb = line / M;
@@ -116,38 +114,39 @@ __device__ __forceinline__ void surface_pass(const StageArgs<M, Real>& a, long l
     for (int h = 0; h < 5; ++h) {
         S0.u[h] = Real(s_u[h][n0]);
         S1.u[h] = Real(s_u[h][n1]);
-        Nm.u[h] = Real(fn.m[D][h]);
-        Np.u[h] = Real(fn.p[D][h]);
+        Nm.u[h] = Real(um[h]);
+        Np.u[h] = Real(up[h]);
     }
     if constexpr (F32) {
         S0.p64 = s_p64[n0];
         S1.p64 = s_p64[n1];
-        Nm.p64 = pressure(a.ph64.gas, fn.m[D]);
-        Np.p64 = pressure(a.ph64.gas, fn.p[D]);
-        // neighbours inside the block: their staged nodes in LDS
-        const long long em = geo.nbr[2 * D], ep = geo.nbr[2 * D + 1];
-        const bool im = valid && in_block(em, e0, a.nelem, BE);
-        const bool ip = valid && in_block(ep, e0, a.nelem, BE);
-        const int nm = bslot<M>((im ? int(em - e0) : 0) * M3, nidx<D, M>(M - 1, ta, tb));
-        const int np = bslot<M>((ip ? int(ep - e0) : 0) * M3, nidx<D, M>(0, ta, tb));
+        Nm.p64 = pressure(a.ph64.gas, um);
+        Np.p64 = pressure(a.ph64.gas, up);
+        if constexpr (INBLK) {
+            // neighbours inside the block: their staged nodes in LDS
+            const long long em = geo.nbr[2 * D], ep = geo.nbr[2 * D + 1];
+            const bool im = valid && in_block(em, e0, a.nelem, BE);
+            const bool ip = valid && in_block(ep, e0, a.nelem, BE);
+            const int nm = bslot<M>((im ? int(em - e0) : 0) * M3, nidx<D, M>(M - 1, ta, tb));
+            const int np = bslot<M>((ip ? int(ep - e0) : 0) * M3, nidx<D, M>(0, ta, tb));
 #pragma unroll
-        for (int h = 0; h < 5; ++h) {
-            const Real lm = Real(s_u[h][nm]), lp = Real(s_u[h][np]);
-            Nm.u[h] = im ? lm : Nm.u[h];
-            Np.u[h] = ip ? lp : Np.u[h];
+            for (int h = 0; h < 5; ++h) {
+                const Real lm = Real(s_u[h][nm]), lp = Real(s_u[h][np]);
+                Nm.u[h] = im ? lm : Nm.u[h];
+                Np.u[h] = ip ? lp : Np.u[h];
+            }
+            const double qm = s_p64[nm], qp = s_p64[np];
+            Nm.p64 = im ? qm : Nm.p64;
+            Np.p64 = ip ? qp : Np.p64;
         }
-        const double qm = s_p64[nm], qp = s_p64[np];
-        Nm.p64 = im ? qm : Nm.p64;
-        Np.p64 = ip ? qp : Np.p64;
     }
     make_state<D, false>(g, S0);
     make_state<D, false>(g, S1);
     make_state<D, false>(g, Nm);
     make_state<D, false>(g, Np);
-    Real fm[5], fp[5];
     riemann<SURF, D>(g, Nm, S0, fm);
     riemann<SURF, D>(g, S1, Np, fp);
-    Real jac = Real(0);
+    jac = Real(0);
     if (valid) {
         const long long em = geo.nbr[2 * D];
         const long long ep = geo.nbr[2 * D + 1];
@@ -163,6 +162,24 @@ __device__ __forceinline__ void surface_pass(const StageArgs<M, Real>& a, long l
             for (int h = 0; h < 5; ++h) fp[h] = Real(mf[h * M2]);
         }
     }
+}
+
+// Surface term of direction D: the face fluxes lifted to the end nodes of the
+// line, +jac f*_- / w_0 and -jac f*_+ / w_{M-1}.  With LGL subcells the DG and
+// FV surface terms are the same, so the term does not depend on the blending
+// factor and is added to the accumulators before the volume passes (pass
+// D = 0 initialises them).
+template <int D, int M, int BE, typename Real>
+__device__ __forceinline__ void surface_add(const StageArgs<M, Real>& a, int tid, Real (*s_acc)[BE * M * M * M],
+                                            const Real (&fm)[5], const Real (&fp)[5], Real jac) {
+    using Sh = StageShape<M, BE>;
+    constexpr int M2 = Sh::M2, M3 = Sh::M3;
+    const int el = tid / M2;
+    const int line = tid - el * M2;
+    const int ta = line % M, tb = line / M;
+    const int base = el * M3;
+    const int n0 = bslot<M>(base, nidx<D, M>(0, ta, tb));
+    const int n1 = bslot<M>(base, nidx<D, M>(M - 1, ta, tb));
     const Real cm = jac * a.op.inv_w[0];
     const Real cp = -jac * a.op.inv_w[M - 1];
     if constexpr (D == 0) {
@@ -181,6 +198,16 @@ __device__ __forceinline__ void surface_pass(const StageArgs<M, Real>& a, long l
     }
 }
 
+template <int D, int M, int BE, int SURF, typename Real, typename TU>
+__device__ __forceinline__ void surface_pass(const StageArgs<M, Real>& a, long long e0, const TU (*s_u)[BE * M * M * M],
+                                             Real (*s_acc)[BE * M * M * M], const double* s_p64, const ElemGeom& geo,
+                                             const FaceNodes& fn) {
+    const int tid = threadIdx.x;
+    Real fm[5], fp[5], jac;
+    surface_fluxes<D, M, BE, SURF, true, Real, TU>(a, tid, e0, s_u, s_p64, geo, fn.m[D], fn.p[D], fm, fp, jac);
+    surface_add<D, M, BE, Real>(a, tid, s_acc, fm, fp, jac);
+}
+
 // LSRK update done by the last volume pass itself (x last): the register
 // values of the thread's x-line nodes and the time step in, the new state
 // of those nodes out.
@@ -191,51 +218,12 @@ struct XUpdate {
     double unew[5][M];
 };
 
-// Volume pass of direction D: the thread's M line nodes become node states
-// once; the M(M-1)/2 two-point fluxes (or the weak-form derivative) and the
-// M-1 interior FV interface fluxes read those states.  Only LDS is read.
-// With XUPD and fuse set (FP64, LSRK, pass x run last) the pass does not
-// store its contributions: it adds them to the accumulated surface and y/z
-// terms and applies the LSRK probe to its own line's nodes (register out to
-// HBM, new state into xu), with the same arithmetic as the separate update.
-// Without fuse it stores them like the other passes.  NEAR1: the caller has
-// found every ratio of two densities and of two betas of the block in
-// [sqrt(1/2), sqrt(2)) (ec_flux).
-template <int D, int M, int BE, int VOL, int SURF, typename Real, typename TU, bool XUPD = false, bool NEAR1 = false>
-__device__ __forceinline__ void direction_pass(const StageArgs<M, Real>& a, long long e0, const TU (*s_u)[BE * M * M * M],
-                                               Real (*s_acc)[BE * M * M * M], const Real alpha,
-                                               const double* s_p64, const ElemGeom& geo,
-                                               XUpdate<M>* xu = nullptr, bool fuse = false) {
-    using Sh = StageShape<M, BE>;
-    constexpr int M2 = Sh::M2, M3 = Sh::M3;
-    constexpr bool BETA = (VOL == VOL_EC);
-    const int tid = threadIdx.x;
-    const int el = tid / M2;
-    const int line = tid - el * M2;
-    const int ta = line % M, tb = line / M;
-    const long long e = e0 + el;
-    const bool valid = e < a.nelem;
+// DG volume terms c of a line (direction D) from its node states; jac = 2 / dx
+// and sdx = M / dx, both zero for lanes past the last element.
+template <int D, int M, int VOL, bool NEAR1, typename Real>
+__device__ __forceinline__ void volume_dg(const StageArgs<M, Real>& a, const NodeState<Real> (&S)[M], Real jac, Real sdx,
+                                          Real (&c)[M][5]) {
     const Gas<Real>& g = a.gas;
-    const int base = el * M3;
-
-    constexpr bool F32 = sizeof(Real) == 4;
-    NodeState<Real> S[M];
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-        const int n = bslot<M>(base, nidx<D, M>(i, ta, tb));
-#pragma unroll
-        for (int h = 0; h < 5; ++h) S[i].u[h] = Real(s_u[h][n]);
-        make_state<D, BETA>(g, S[i]);
-        if constexpr (F32) S[i].p64 = s_p64[n];
-    }
-    Real jac = Real(0), sdx = Real(0);
-    if (valid) {
-        const double dx = geo.dx[D];
-        jac = Real(2.0 / dx);
-        sdx = Real(double(M) / dx);
-    }
-
-    Real c[M][5];
     if constexpr (VOL == VOL_WEAK) {
         // 3-D LGL extension of kernel/dgsem/weakform/2d/kernel_flux_mod.f90:242-277:
         // rhs_i = sum_j dgDiff_ij (sdx f_j) here; the surface lifting
@@ -286,7 +274,49 @@ __device__ __forceinline__ void direction_pass(const StageArgs<M, Real>& a, long
 #pragma unroll
             for (int h = 0; h < 5; ++h) c[i][h] = -jac * c[i][h];
     }
+}
 
+// DG volume terms c of line `tid` in direction D, the line's node states S
+// and jac = 2 / dx.
+template <int D, int M, int BE, int VOL, typename Real, typename TU, bool NEAR1>
+__device__ __forceinline__ void volume_terms(const StageArgs<M, Real>& a, int tid, long long e0,
+                                             const TU (*s_u)[BE * M * M * M], const double* s_p64,
+                                             const ElemGeom& geo, NodeState<Real> (&S)[M], Real (&c)[M][5],
+                                             Real& jac) {
+    using Sh = StageShape<M, BE>;
+    constexpr int M2 = Sh::M2, M3 = Sh::M3;
+    constexpr bool BETA = (VOL == VOL_EC);
+    const int el = tid / M2;
+    const int line = tid - el * M2;
+    const int ta = line % M, tb = line / M;
+    const bool valid = e0 + el < a.nelem;
+    const Gas<Real>& g = a.gas;
+    const int base = el * M3;
+
+    constexpr bool F32 = sizeof(Real) == 4;
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+        const int n = bslot<M>(base, nidx<D, M>(i, ta, tb));
+#pragma unroll
+        for (int h = 0; h < 5; ++h) S[i].u[h] = Real(s_u[h][n]);
+        make_state<D, BETA>(g, S[i]);
+        if constexpr (F32) S[i].p64 = s_p64[n];
+    }
+    jac = Real(0);
+    Real sdx = Real(0);
+    if (valid) {
+        const double dx = geo.dx[D];
+        jac = Real(2.0 / dx);
+        sdx = Real(double(M) / dx);
+    }
+    volume_dg<D, M, VOL, NEAR1, Real>(a, S, jac, sdx, c);
+}
+
+// FV subcells of the line blended into its terms with the factor alpha.
+template <int D, int M, int SURF, typename Real>
+__device__ __forceinline__ void blend_fv(const StageArgs<M, Real>& a, const NodeState<Real> (&S)[M], Real jac, Real alpha,
+                                         Real (&c)[M][5]) {
+    const Gas<Real>& g = a.gas;
     // FV subcells on the LGL sub-grid (Hennemann et al. 2021), first order:
     // rhs_i = -jac (F_{i+1/2} - F_{i-1/2}) / w_i, blended as
     // (1-alpha) DG + alpha FV; the element-face fluxes F_{-1/2} = f*_- and
@@ -314,6 +344,37 @@ __device__ __forceinline__ void direction_pass(const StageArgs<M, Real>& a, long
             }
         }
     }
+}
+
+// Volume pass of direction D: the thread's M line nodes become node states
+// once; the M(M-1)/2 two-point fluxes (or the weak-form derivative) and the
+// M-1 interior FV interface fluxes read those states.  Only LDS is read.
+// With XUPD and fuse set (FP64, LSRK, pass x run last) the pass does not
+// store its contributions: it adds them to the accumulated surface and y/z
+// terms and applies the LSRK probe to its own line's nodes (register out to
+// HBM, new state into xu), with the same arithmetic as the separate update.
+// Without fuse it stores them like the other passes.  NEAR1: the caller has
+// found every ratio of two densities and of two betas of the block in
+// [sqrt(1/2), sqrt(2)) (ec_flux).
+template <int D, int M, int BE, int VOL, int SURF, typename Real, typename TU, bool XUPD = false, bool NEAR1 = false>
+__device__ __forceinline__ void direction_pass(const StageArgs<M, Real>& a, long long e0, const TU (*s_u)[BE * M * M * M],
+                                               Real (*s_acc)[BE * M * M * M], const Real alpha,
+                                               const double* s_p64, const ElemGeom& geo,
+                                               XUpdate<M>* xu = nullptr, bool fuse = false) {
+    using Sh = StageShape<M, BE>;
+    constexpr int M2 = Sh::M2, M3 = Sh::M3;
+    const int tid = threadIdx.x;
+    const int el = tid / M2;
+    const int line = tid - el * M2;
+    const int ta = line % M, tb = line / M;
+    const long long e = e0 + el;
+    const bool valid = e < a.nelem;
+    const int base = el * M3;
+
+    NodeState<Real> S[M];
+    Real c[M][5], jac;
+    volume_terms<D, M, BE, VOL, Real, TU, NEAR1>(a, tid, e0, s_u, s_p64, geo, S, c, jac);
+    blend_fv<D, M, SURF, Real>(a, S, jac, alpha, c);
 
     static_assert(!XUPD || sizeof(Real) == 8, "the fused update is the FP64 path's");
     bool fused = false;

@@ -24,73 +24,27 @@ __device__ __forceinline__ void mhd_riemann(const MhdGas<Real>& g, const MhdStat
         mhd_rusanov<D>(g, L, R, f);
 }
 
-template <int D, int M, int BE, int VOL, int SURF, typename Real, typename TU>
-__device__ __forceinline__ void direction_pass_mhd(const StageArgs<M, Real>& a, const MhdGas<Real>& g, long long e0,
-                                                   const TU (*s_u)[BE * M * M * M],
-                                                   Real (*s_acc)[BE * M * M * M], const Real alpha) {
-    using Sh = StageShape<M, BE>;
-    constexpr int M2 = Sh::M2, M3 = Sh::M3, V = 9;
+// Face fluxes of a line with the inner state's non-conservative terms: S the
+// line's node states, Nm and Np the nodes across its ends.
+template <int D, int M, int SURF, typename Real>
+__device__ __forceinline__ void mhd_face_fluxes(const MhdGas<Real>& g, const MhdState<Real> (&S)[M], MhdState<Real>& Nm,
+                                                MhdState<Real>& Np, Real (&fm)[9], Real (&fp)[9]) {
     constexpr int BN = Mag<D, 0>::idx;
-    constexpr bool BETA = (VOL == VOL_EC);
-    const int tid = threadIdx.x;
-    const int el = tid / M2;
-    const int line = tid - el * M2;
-    const int ta = line % M, tb = line / M;
-    const long long e = e0 + el;
-    const bool valid = e < a.nelem;
-    const long long EM3 = a.nelem * (long long)M3;
-    const int base = el * M3;
+    mhd_make_state<false>(g, Nm);
+    mhd_make_state<false>(g, Np);
+    mhd_riemann<SURF, D>(g, Nm, S[0], fm);
+    mhd_riemann<SURF, D>(g, S[M - 1], Np, fp);
+    mhd_nc_add<D>(g, S[0], Real(0.5) * (Nm.u[BN] + S[0].u[BN]), Real(0.5) * (Nm.u[GLMP] + S[0].u[GLMP]), fm);
+    mhd_nc_add<D>(g, S[M - 1], Real(0.5) * (S[M - 1].u[BN] + Np.u[BN]), Real(0.5) * (S[M - 1].u[GLMP] + Np.u[GLMP]),
+                  fp);
+}
 
-    MhdState<Real> S[M];
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-        const int n = bslot<M>(base, nidx<D, M>(i, ta, tb));
-#pragma unroll
-        for (int h = 0; h < V; ++h) S[i].u[h] = Real(s_u[h][n]);
-        mhd_make_state<BETA>(g, S[i]);
-    }
-    Real fm[V], fp[V];
-    // Lanes past the last element read element 0's neighbours (their results
-    // are discarded): unconditional loads, so later loads need not wait.
-    const long long ec = valid ? e : 0;
-    const Real jac = Real(2.0 / a.delta[ec * 3 + D]);
-    {
-        // A face on a non-conforming interface takes its flux, with this
-        // side's non-conservative term, from the mortar pass: the face
-        // computation then runs on the element's own face node and is
-        // discarded.
-        const long long em = a.nbr[ec * 6 + 2 * D];
-        const long long ep = a.nbr[ec * 6 + 2 * D + 1];
-        MhdState<Real> Nm, Np;
-        {
-            const double* um = a.u_in + (em < 0 ? ec * M3 + nidx<D, M>(0, ta, tb) : em * M3 + nidx<D, M>(M - 1, ta, tb));
-            const double* up = a.u_in + (ep < 0 ? ec * M3 + nidx<D, M>(M - 1, ta, tb) : ep * M3 + nidx<D, M>(0, ta, tb));
-#pragma unroll
-            for (int h = 0; h < V; ++h) {
-                Nm.u[h] = Real(um[h * EM3]);
-                Np.u[h] = Real(up[h * EM3]);
-            }
-        }
-        mhd_make_state<false>(g, Nm);
-        mhd_make_state<false>(g, Np);
-        mhd_riemann<SURF, D>(g, Nm, S[0], fm);
-        mhd_riemann<SURF, D>(g, S[M - 1], Np, fp);
-        mhd_nc_add<D>(g, S[0], Real(0.5) * (Nm.u[BN] + S[0].u[BN]), Real(0.5) * (Nm.u[GLMP] + S[0].u[GLMP]), fm);
-        mhd_nc_add<D>(g, S[M - 1], Real(0.5) * (S[M - 1].u[BN] + Np.u[BN]),
-                      Real(0.5) * (S[M - 1].u[GLMP] + Np.u[GLMP]), fp);
-        if (em < 0) {
-            const double* mf = a.mortar_flux + size_t(-em - 1) * V * M2 + ta + M * tb;
-#pragma unroll
-            for (int h = 0; h < V; ++h) fm[h] = Real(mf[h * M2]);
-        }
-        if (ep < 0) {
-            const double* mf = a.mortar_flux + size_t(-ep - 1) * V * M2 + ta + M * tb;
-#pragma unroll
-            for (int h = 0; h < V; ++h) fp[h] = Real(mf[h * M2]);
-        }
-    }
-
-    Real c[M][V];
+// DG terms c of a line: volume and face terms; jac = 2 / dx.
+template <int D, int M, int VOL, typename Real>
+__device__ __forceinline__ void mhd_volume_dg(const StageArgs<M, Real>& a, const MhdGas<Real>& g,
+                                              const MhdState<Real> (&S)[M], const Real (&fm)[9], const Real (&fp)[9],
+                                              Real jac, Real (&c)[M][9]) {
+    constexpr int V = 9, BN = Mag<D, 0>::idx;
     {
         Real sB[M], sG[M];
 #pragma unroll
@@ -133,7 +87,14 @@ __device__ __forceinline__ void direction_pass_mhd(const StageArgs<M, Real>& a, 
     for (int i = 0; i < M; ++i)
 #pragma unroll
         for (int h = 0; h < V; ++h) c[i][h] = -jac * c[i][h];
+}
 
+// FV subcells blended into the line's terms.
+template <int D, int M, int SURF, typename Real>
+__device__ __forceinline__ void mhd_blend_fv(const StageArgs<M, Real>& a, const MhdGas<Real>& g,
+                                             const MhdState<Real> (&S)[M], const Real (&fm)[9], const Real (&fp)[9],
+                                             Real jac, Real alpha, Real (&c)[M][9]) {
+    constexpr int V = 9, BN = Mag<D, 0>::idx;
     // FV subcells on the LGL sub-grid with the non-conservative terms per
     // interface side: cell i gets Phi(u_i) ({{.}}_{i+1/2} - {{.}}_{i-1/2}),
     // the element faces already carry theirs in fm/fp.
@@ -169,6 +130,68 @@ __device__ __forceinline__ void direction_pass_mhd(const StageArgs<M, Real>& a, 
             Gl = Gr;
         }
     }
+}
+
+template <int D, int M, int BE, int VOL, int SURF, typename Real, typename TU>
+__device__ __forceinline__ void direction_pass_mhd(const StageArgs<M, Real>& a, const MhdGas<Real>& g, long long e0,
+                                                   const TU (*s_u)[BE * M * M * M],
+                                                   Real (*s_acc)[BE * M * M * M], const Real alpha) {
+    using Sh = StageShape<M, BE>;
+    constexpr int M2 = Sh::M2, M3 = Sh::M3, V = 9;
+    constexpr bool BETA = (VOL == VOL_EC);
+    const int tid = threadIdx.x;
+    const int el = tid / M2;
+    const int line = tid - el * M2;
+    const int ta = line % M, tb = line / M;
+    const long long e = e0 + el;
+    const bool valid = e < a.nelem;
+    const long long EM3 = a.nelem * (long long)M3;
+    const int base = el * M3;
+
+    MhdState<Real> S[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+        const int n = bslot<M>(base, nidx<D, M>(i, ta, tb));
+#pragma unroll
+        for (int h = 0; h < V; ++h) S[i].u[h] = Real(s_u[h][n]);
+        mhd_make_state<BETA>(g, S[i]);
+    }
+    // Lanes past the last element read element 0's neighbours (their results
+    // are discarded): unconditional loads, so later loads need not wait.
+    const long long ec = valid ? e : 0;
+    const Real jac = Real(2.0 / a.delta[ec * 3 + D]);
+    Real fm[V], fp[V], c[M][V];
+    {
+        // A face on a non-conforming interface takes its flux, with this
+        // side's non-conservative term, from the mortar pass: the face
+        // computation then runs on the element's own face node and is
+        // discarded.
+        const long long em = a.nbr[ec * 6 + 2 * D];
+        const long long ep = a.nbr[ec * 6 + 2 * D + 1];
+        MhdState<Real> Nm, Np;
+        {
+            const double* um = a.u_in + (em < 0 ? ec * M3 + nidx<D, M>(0, ta, tb) : em * M3 + nidx<D, M>(M - 1, ta, tb));
+            const double* up = a.u_in + (ep < 0 ? ec * M3 + nidx<D, M>(M - 1, ta, tb) : ep * M3 + nidx<D, M>(0, ta, tb));
+#pragma unroll
+            for (int h = 0; h < V; ++h) {
+                Nm.u[h] = Real(um[h * EM3]);
+                Np.u[h] = Real(up[h * EM3]);
+            }
+        }
+        mhd_face_fluxes<D, M, SURF, Real>(g, S, Nm, Np, fm, fp);
+        if (em < 0) {
+            const double* mf = a.mortar_flux + size_t(-em - 1) * V * M2 + ta + M * tb;
+#pragma unroll
+            for (int h = 0; h < V; ++h) fm[h] = Real(mf[h * M2]);
+        }
+        if (ep < 0) {
+            const double* mf = a.mortar_flux + size_t(-ep - 1) * V * M2 + ta + M * tb;
+#pragma unroll
+            for (int h = 0; h < V; ++h) fp[h] = Real(mf[h * M2]);
+        }
+    }
+    mhd_volume_dg<D, M, VOL, Real>(a, g, S, fm, fp, jac, c);
+    mhd_blend_fv<D, M, SURF, Real>(a, g, S, fm, fp, jac, alpha, c);
 
 #pragma unroll
     for (int i = 0; i < M; ++i) {

@@ -44,11 +44,10 @@ namespace nemo {
 // the cancellation in tot - c1 or c1 - c2 when the high modes are small.
 // q must be complete (barrier) on entry; t1 and t2 are work rows; t1 is
 // free again on return, t2 only after a barrier.
-template <int M, int BE, typename Real>
-__device__ __forceinline__ void modal_partials(const StageArgs<M, Real>& a, const Real* q, Real* t1, Real* t2,
+template <int M, int BE, bool SHARED, typename Real>
+__device__ __forceinline__ void modal_partials(const StageArgs<M, Real>& a, int tid, const Real* q, Real* t1, Real* t2,
                                                Real& tot, Real& c1, Real& s1, Real& sh2) {
     constexpr int M2 = M * M, M3 = M2 * M;
-    const int tid = threadIdx.x;
     const int el = tid / M2, line = tid - el * M2;
     const int ta = line % M, tb = line / M;
     const int base = el * M3;
@@ -64,7 +63,7 @@ __device__ __forceinline__ void modal_partials(const StageArgs<M, Real>& a, cons
             t1[bslot<M>(base, r + M * ta + M2 * tb)] = s;
         }
     }
-    __syncthreads();
+    wave_sync<SHARED>();
     {  // y: t2(i,b,k) = sum_j Vinv(b,j) t1(i,j,k)
         Real v[M];
 #pragma unroll
@@ -77,7 +76,7 @@ __device__ __forceinline__ void modal_partials(const StageArgs<M, Real>& a, cons
             t2[bslot<M>(base, ta + M * r + M2 * tb)] = s;
         }
     }
-    __syncthreads();
+    wave_sync<SHARED>();
     {  // z: modal(a,b,c) = sum_k Vinv(c,k) t2(a,b,k); energies
         Real v[M];
 #pragma unroll
@@ -126,14 +125,13 @@ __device__ __forceinline__ double pp_alpha(const StageArgs<M, Real>& a, Real tot
 // Returns the blending factor of the calling thread's element (one
 // workgroup is one wavefront, so it is broadcast by a lane shuffle); with
 // write_out the factor also goes to alpha_out.
-template <int EQ, int M, int BE, typename Real, typename TU>
-__device__ __forceinline__ Real indicator_pp(const StageArgs<M, Real>& a, long long e0,
+template <int EQ, int M, int BE, typename Real, typename TU, bool SHARED = false>
+__device__ __forceinline__ Real indicator_pp(const StageArgs<M, Real>& a, int tid, long long e0,
                                              const TU (*s_u)[BE * M * M * M], Real (*s_acc)[BE * M * M * M],
                                              const double* s_p64, bool write_out = true) {
     constexpr int V = NVars<EQ>::V;
     using Sh = StageShape<M, BE>;
     constexpr int M2 = Sh::M2, NN = Sh::NN, NT = Sh::NT;
-    const int tid = threadIdx.x;
     Real* q = s_acc[2];
     for (int idx = tid; idx < NN; idx += NT) {
         const int sl = slot<M>(idx);
@@ -146,16 +144,16 @@ __device__ __forceinline__ Real indicator_pp(const StageArgs<M, Real>& a, long l
             q[sl] = Real(uu[DENS] * pressure64<EQ>(a.ph64, uu));
         }
     }
-    __syncthreads();
+    wave_sync<SHARED>();
     Real tot, c1, s1, sh2;
-    modal_partials<M, BE, Real>(a, q, s_acc[0], s_acc[1], tot, c1, s1, sh2);
+    modal_partials<M, BE, SHARED, Real>(a, tid, q, s_acc[0], s_acc[1], tot, c1, s1, sh2);
     // rows 0 (t1) and 2 (q) are dead after the y contraction; rows 0, 2..4
     // take the partials
     s_acc[0][tid] = tot;
     s_acc[2][tid] = s1;
     s_acc[3][tid] = c1;
     s_acc[4][tid] = sh2;
-    __syncthreads();
+    wave_sync<SHARED>();
     const int el = tid / M2, line = tid - el * M2;
     Real alpha_el = Real(0);
     if (line == 0) {
@@ -172,7 +170,7 @@ __device__ __forceinline__ Real indicator_pp(const StageArgs<M, Real>& a, long l
         if (write_out && a.alpha_out && e < a.nelem) a.alpha_out[e] = alpha;
     }
     alpha_el = __shfl(alpha_el, el * M2);
-    __syncthreads();  // the work rows are the direction passes' accumulators
+    wave_sync<SHARED>();  // the work rows are the direction passes' accumulators
     return alpha_el;
 }
 
@@ -204,14 +202,13 @@ __device__ __forceinline__ uint32_t sample_hash(long long e, uint32_t step) {
 // any node has rho <= 0 or p <= 0, the PP factor is used.  The factor is
 // kept in alpha_step for the remaining stages of the step.  With feat_out
 // (training data) it writes the features and the PP factor of every element.
-template <int EQ, int M, int BE, typename Real, typename TU>
-__device__ __forceinline__ Real indicator_mlp(const StageArgs<M, Real>& a, long long e0,
+template <int EQ, int M, int BE, typename Real, typename TU, bool SHARED = false>
+__device__ __forceinline__ Real indicator_mlp(const StageArgs<M, Real>& a, int tid, long long e0,
                                               const TU (*s_u)[BE * M * M * M], Real (*s_acc)[BE * M * M * M],
                                               const double* s_p64) {
     static_assert(M == 4 && BE * M * M == 64, "the learned indicator maps 16 lanes to an element");
     constexpr int V = NVars<EQ>::V;
     constexpr int M2 = 16, NN = BE * 64, NT = 64;
-    const int tid = threadIdx.x;
     const int el = tid / M2;
     const long long e = e0 + el;
     const bool valid = e < a.nelem;
@@ -238,9 +235,9 @@ __device__ __forceinline__ Real indicator_mlp(const StageArgs<M, Real>& a, long 
             q[sl] = Real(pass == 0 ? rho : p);
             if (pass == 0 && !(rho > 0.0 && p > 0.0) && e0 + idx / 64 < a.nelem) bad |= 1u << (idx / 64);
         }
-        __syncthreads();
+        wave_sync<SHARED>();
         Real tot, c1, s1, sh2;
-        modal_partials<M, BE, Real>(a, q, s_acc[0], s_acc[1], tot, c1, s1, sh2);
+        modal_partials<M, BE, SHARED, Real>(a, tid, q, s_acc[0], s_acc[1], tot, c1, s1, sh2);
         Real s2 = s1 + sh2;  // top two shells
         tot = sum16(tot);
         s1 = sum16(s1);
@@ -254,7 +251,7 @@ __device__ __forceinline__ Real indicator_mlp(const StageArgs<M, Real>& a, long 
             fp1 = f1;
             fp2 = f2;
         }
-        __syncthreads();
+        wave_sync<SHARED>();
     }
     const float x[4] = {mlp_feature(fr1), mlp_feature(fr2), mlp_feature(fp1), mlp_feature(fp2)};
     uint32_t bad_el = 0;
@@ -270,7 +267,7 @@ __device__ __forceinline__ Real indicator_mlp(const StageArgs<M, Real>& a, long 
     const bool judged = valid && (a.feat_out || sample_hash(e0, a.step_index) < a.sample_thresh);
     const bool need_pp = __any(judged) || bad_el != 0;
     Real a_pp = Real(0);
-    if (need_pp) a_pp = indicator_pp<EQ, M, BE, Real, TU>(a, e0, s_u, s_acc, s_p64, false);
+    if (need_pp) a_pp = indicator_pp<EQ, M, BE, Real, TU, SHARED>(a, tid, e0, s_u, s_acc, s_p64, false);
 
     if (a.feat_out) {  // training data: features and PP factor of every element
         if ((tid & 15) == 0 && valid) {
@@ -672,12 +669,12 @@ __device__ __forceinline__ void stage_block(const StageArgs<M, Real>& a, const l
 
     Real alpha = Real(0);
     if constexpr (IK == IK_MLP) {
-        alpha = indicator_mlp<EQ, M, BE, Real, TU>(a, e0, s_u, s_acc, s_p64);
+        alpha = indicator_mlp<EQ, M, BE, Real, TU>(a, tid, e0, s_u, s_acc, s_p64);
     } else if constexpr (IK == IK_STORED) {
         const long long e = e0 + tid / Sh::M2;
         alpha = e < a.nelem ? Real(a.alpha_step[e]) : Real(0);
     } else if (a.indicator == IND_PP) {
-        alpha = indicator_pp<EQ, M, BE, Real, TU>(a, e0, s_u, s_acc, s_p64);
+        alpha = indicator_pp<EQ, M, BE, Real, TU>(a, tid, e0, s_u, s_acc, s_p64);
     }
 
     // indicator only (nemo_gpu_indicator, Euler): the factor has gone to
