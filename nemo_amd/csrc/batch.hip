@@ -163,8 +163,9 @@ void launch_group_stage(Batch* b, Group& gr, int stage, bool cfl) {
 template <int M>
 void launch_group_cfl(Batch* b, Group& gr) {
     constexpr int BE = Tile<M>::BE;
-    hipLaunchKernelGGL((nemo::cfl_kernel<nemo::EQ_EULER, M, BE>), dim3(unsigned(gr.nblocks)), dim3(BE * M * M), 0,
-                       b->stream, gr.u[gr.cur], gr.delta, gr.nelem, make_phys64(b->cfg), b->part + 4 * gr.part_off);
+    hipLaunchKernelGGL((nemo::cfl_kernel<nemo::EQ_EULER, M, BE>), dim3(unsigned(gr.nblocks)), dim3(nemo::CFL_NT), 0,
+                       b->stream, gr.u[gr.cur], gr.delta, gr.nelem, make_phys64(b->cfg), b->part + 4 * gr.part_off,
+                       nemo::CflFinal{});
 }
 
 // Per-run reduction of the block partials (one workgroup per run, fixed

@@ -73,6 +73,16 @@ __device__ __forceinline__ double lambda_max64(const Phys64& P, const double* u)
         return lambda_max<D>(P.gas, u);
 }
 
+// Where the time step of the CFL reduction goes.
+struct CflFinal {
+    double* dt_dev;        // dt, lmax, vmax, GLM c_h, GLM alpha
+    double* hist;          // optional history of time steps, and its slot
+    long long slot;
+    double* host;          // optional pinned host memory: dt, lmax, vmax
+    unsigned int* ticket;  // blocks that have written their partial; null: a separate reduction follows
+    double cfl;
+};
+
 template <int M, typename Real>
 struct StageArgs {
     const double* __restrict__ u_in;
@@ -89,7 +99,8 @@ struct StageArgs {
     const double* __restrict__ dt_run;     // batched ensemble: time step per run
     const int32_t* __restrict__ block_run; // batched ensemble: run of each block
     int* __restrict__ status;
-    double* __restrict__ cfl_part;   // non-null: per-block CFL partials of the new state
+    double* cfl_part;                // non-null: per-block CFL partials of the new state
+    CflFinal fin;                    // small-mesh form: the last block reduces the partials
     // learned indicator
     const float* __restrict__ mlp;   // network parameters, inference layout
     double* __restrict__ alpha_step; // per element factor of the current step

@@ -944,7 +944,7 @@ __device__ __forceinline__ void stage_block(const StageArgs<M, Real>& a, const l
                 double* su[V];
 #pragma unroll
                 for (int h = 0; h < V; ++h) su[h] = s_u64[h];
-                if (!repair_element<EQ, M>(a.ph64, a.rk.w64, su, tid * M3)) atomicOr(a.status, 1);
+                if (!repair_element<EQ, M>(a.ph64, a.rk.w64, su, tid * M3)) *(volatile int*)a.status = 1;
             }
             __syncthreads();
         }
@@ -1018,33 +1018,11 @@ __global__ __launch_bounds__(BE * M * M) void stage_kernel_persistent(StageArgs<
     }
 }
 
-// Standalone CFL reduction of a state in HBM (first step, calc_timestep):
-// the same per-block partials as the fused stage epilogue.
-template <int EQ, int M, int BE>
-__global__ __launch_bounds__(BE * M * M) void cfl_kernel(const double* __restrict__ u, const double* __restrict__ delta,
-                                                         long long nelem, Phys64 P, double* __restrict__ part) {
-    constexpr int M3 = M * M * M, NN = BE * M3, NT = BE * M * M, V = NVars<EQ>::V;
-    __shared__ double s_u[V][NN];
-    __shared__ double s_w[4][NT];
-    const int tid = threadIdx.x;
-    const long long blk = blockIdx.x;
-    const long long e0 = blk * BE;
-    const long long EM3 = nelem * (long long)M3;
-    const long long nvalid = (nelem - e0 < BE ? nelem - e0 : BE) * (long long)M3;
-#pragma unroll
-    for (int h = 0; h < V; ++h)
-        for (int idx = tid; idx < NN; idx += NT)
-            s_u[h][slot<M>(idx)] = idx < nvalid ? u[h * EM3 + e0 * M3 + idx] : (h == 0 || h == 4 ? 1.0 : 0.0);
-    __syncthreads();
-    block_cfl<EQ, M, BE, NT>(P, delta, e0, nelem, s_u, &s_w[0][0], part + 4 * blk);
-}
-
 // Deterministic reduction of the per-block partials (min and max are exact,
 // so the result does not depend on the order) and
 // dt = 0.5*CFL/(2*N_NODES-1) * dtmin (kernel_timestep_mod.f90:49); for
 // GLM-MHD also c_h = 2|lmax - vmax| and alpha = c_h/0.18
 // (kernel/mcfv/3d/kernel_timestep_mod.f90:53-56).
-// dt_dev: [0] dt, [1] lmax, [2] vmax, [3] c_h, [4] alpha.
 // Two levels: block i of a grid of G <= CFL_GRID blocks reduces the i-th
 // contiguous G-th of the block partials (3 of the 4 values each: dt
 // candidate, lmax, vmax) into red[i]; the block that finishes last (ticket) reduces red and
@@ -1071,10 +1049,24 @@ __device__ __forceinline__ void cfl_block_reduce(double& dt, double& lm, double&
     vm = s[2][0];
 }
 
-static __global__ __launch_bounds__(CFL_NT) void cfl_finalize(const double* __restrict__ part, long long npart,
-                                                              double cfl, int M, double* __restrict__ dt_dev,
-                                                              double* __restrict__ hist, long long slot,
-                                                              double* __restrict__ red, unsigned int* __restrict__ ticket) {
+__device__ __forceinline__ void cfl_store(const CflFinal& f, int M, double dtmin, double lm, double vm) {
+    const double d = 0.5 * f.cfl / double(2 * M - 1) * dtmin;
+    f.dt_dev[0] = d;
+    f.dt_dev[1] = lm;
+    f.dt_dev[2] = vm;
+    const double ch = 2.0 * fabs(lm - vm);
+    f.dt_dev[3] = ch;
+    f.dt_dev[4] = ch / 0.18;
+    if (f.hist && f.slot >= 0) f.hist[f.slot] = d;
+    if (f.host) {
+        f.host[0] = d;
+        f.host[1] = lm;
+        f.host[2] = vm;
+    }
+}
+
+static __global__ __launch_bounds__(CFL_NT) void cfl_finalize(const double* __restrict__ part, long long npart, int M,
+                                                              CflFinal fin, double* __restrict__ red) {
     __shared__ double s[3][CFL_NT];
     __shared__ bool last;
     const int tid = threadIdx.x;
@@ -1094,7 +1086,7 @@ static __global__ __launch_bounds__(CFL_NT) void cfl_finalize(const double* __re
         red[3 * blockIdx.x + 1] = lm;
         red[3 * blockIdx.x + 2] = vm;
         __threadfence();
-        last = atomicAdd(ticket, 1u) == unsigned(G - 1);
+        last = atomicAdd(fin.ticket, 1u) == unsigned(G - 1);
     }
     __syncthreads();
     if (!last) return;
@@ -1109,16 +1101,128 @@ static __global__ __launch_bounds__(CFL_NT) void cfl_finalize(const double* __re
     }
     cfl_block_reduce(dt, lm, vm, s);
     if (tid == 0) {
-        const double d = 0.5 * cfl / double(2 * M - 1) * dt;
-        dt_dev[0] = d;
-        dt_dev[1] = lm;
-        dt_dev[2] = vm;
-        const double ch = 2.0 * fabs(lm - vm);
-        dt_dev[3] = ch;
-        dt_dev[4] = ch / 0.18;
-        if (hist && slot >= 0) hist[slot] = d;
-        *ticket = 0u;
+        cfl_store(fin, M, dt, lm, vm);
+        *fin.ticket = 0u;
     }
+}
+
+// CFL partial of a block of elements, one node (new state st) per thread of
+// 256: maxima over the element's nodes as LDS maxima of the bit patterns (all
+// values are >= 0; a NaN counts as 0, as in block_cfl's comparisons).  s_max
+// (4 values per element) is zero on entry, a barrier before.
+template <int EQ, int M, int BE>
+__device__ __forceinline__ void block_cfl_nodes(const Phys64& P, const double* __restrict__ delta, long long e0,
+                                                long long nelem, bool own, const double* st,
+                                                unsigned long long* s_max, double* out) {
+    constexpr int M3 = M * M * M;
+    const int tid = threadIdx.x;
+    if (own) {
+        unsigned long long* m = s_max + 4 * (tid / M3);
+        auto put = [&](int k, double x) {
+            if (x > 0.0) atomicMax(&m[k], (unsigned long long)__double_as_longlong(x));
+        };
+        put(0, lambda_max64<EQ, 0>(P, st));
+        put(1, lambda_max64<EQ, 1>(P, st));
+        put(2, lambda_max64<EQ, 2>(P, st));
+        const double v0 = fabs(st[1] / st[0]), v1 = fabs(st[2] / st[0]), v2 = fabs(st[3] / st[0]);
+        double v = v0 > v1 ? v0 : v1;
+        v = v > v2 ? v : v2;
+        put(3, v);
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double dtb = 1.7976931348623157e308, lmb = 0.0, vmb = 0.0;
+        for (int k = 0; k < BE && e0 + k < nelem; ++k) {
+            const long long e = e0 + k;
+            const double m0 = __longlong_as_double((long long)s_max[4 * k + 0]);
+            const double m1 = __longlong_as_double((long long)s_max[4 * k + 1]);
+            const double m2 = __longlong_as_double((long long)s_max[4 * k + 2]);
+            const double vm = __longlong_as_double((long long)s_max[4 * k + 3]);
+            const double t0 = delta[e * 3 + 0] / m0, t1 = delta[e * 3 + 1] / m1, t2 = delta[e * 3 + 2] / m2;
+            double dte = t0 < t1 ? t0 : t1;
+            dte = dte < t2 ? dte : t2;
+            double lme = m0 > m1 ? m0 : m1;
+            lme = lme > m2 ? lme : m2;
+            dtb = dte < dtb ? dte : dtb;
+            lmb = lme > lmb ? lme : lmb;
+            vmb = vm > vmb ? vm : vmb;
+        }
+        // device-scope stores, which leave no dirty line in this XCD's L2
+        // (cfl_last_block)
+        __hip_atomic_store(out + 0, dtb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(out + 1, lmb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(out + 2, vmb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// Up to this many blocks the one that finishes last reduces the partials of
+// all (eight loads per thread, all in flight at once), and the reduction needs
+// no launch of its own (7 us and a gap, against 11 us for a whole stage of 8^3
+// elements; more partials would be read in several rounds by one CU).
+constexpr int CFL_FUSE = 2048;
+
+// The end of a launch of `grid` blocks of CFL_NT threads, each of which has
+// written its partial (thread 0, device-scope stores): the last one reduces
+// them and rearms the ticket.  Thread 0 waits for its own stores and draws the
+// ticket; the partials are read with device-scope loads.  A device-scope fence
+// would write back the XCD's whole L2, which holds the new state, once per
+// block (743 blocks: 17 us of a 26 us stage).
+__device__ __forceinline__ void cfl_last_block(const double* part, int grid, const CflFinal& fin, int M,
+                                               double (*s)[CFL_NT], int* s_last) {
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        *s_last = __hip_atomic_fetch_add(fin.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                  unsigned(grid - 1);
+    }
+    __syncthreads();
+    if (!*s_last) return;
+    constexpr int K = CFL_FUSE / CFL_NT;
+    double q[K][3];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int i = tid + k * CFL_NT < grid ? tid + k * CFL_NT : 0;  // (min and max: a repeat changes nothing)
+#pragma unroll
+        for (int h = 0; h < 3; ++h)
+            q[k][h] = __hip_atomic_load(part + 4 * (long long)i + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    double dt = q[0][0], lm = q[0][1], vm = q[0][2];
+#pragma unroll
+    for (int k = 1; k < K; ++k) {
+        dt = q[k][0] < dt ? q[k][0] : dt;
+        lm = q[k][1] > lm ? q[k][1] : lm;
+        vm = q[k][2] > vm ? q[k][2] : vm;
+    }
+    cfl_block_reduce(dt, lm, vm, s);
+    if (tid == 0) {
+        cfl_store(fin, M, dt, lm, vm);
+        *fin.ticket = 0u;
+    }
+}
+
+// Standalone CFL reduction of a state in HBM (first step, calc_timestep): the
+// same per-block partials as the stage kernels' epilogues, a node per thread.
+// Bound by the read of the state (64^3, 671 MB: 331 us with one wavefront per
+// block and the block staged in LDS, 252 us now).
+template <int EQ, int M, int BE>
+__global__ __launch_bounds__(CFL_NT) void cfl_kernel(const double* __restrict__ u, const double* __restrict__ delta,
+                                                     long long nelem, Phys64 P, double* part, CflFinal fin) {
+    constexpr int M3 = M * M * M, V = NVars<EQ>::V;
+    static_assert(BE * M3 <= CFL_NT, "a node per thread");
+    __shared__ double s[3][CFL_NT];
+    __shared__ unsigned long long s_max[4 * BE];
+    __shared__ int s_last;
+    const int tid = threadIdx.x;
+    const long long e0 = blockIdx.x * (long long)BE;
+    const long long EM3 = nelem * (long long)M3;
+    const bool own = tid < int(nelem - e0 < BE ? nelem - e0 : BE) * M3;
+    double st[V];
+#pragma unroll
+    for (int h = 0; h < V; ++h) st[h] = u[h * EM3 + (own ? e0 * M3 + tid : 0)];
+    if (tid < 4 * BE) s_max[tid] = 0ull;
+    __syncthreads();
+    block_cfl_nodes<EQ, M, BE>(P, delta, e0, nelem, own, st, s_max, part + 4 * (long long)blockIdx.x);
+    if (fin.ticket) cfl_last_block(part, int(gridDim.x), fin, M, s, &s_last);
 }
 
 }  // namespace nemo

@@ -18,7 +18,7 @@
 
 namespace nemo {
 
-constexpr int WIDE_NT = 256;
+constexpr int WIDE_NT = CFL_NT;
 
 // Variable in row h of a state rotated to direction d.
 __device__ __forceinline__ int rotated_row(int h, int d) {
@@ -33,6 +33,7 @@ __device__ __forceinline__ void stage_block_wide(const StageArgs<M, Real>& a, co
     using TU = typename L::TU;
     constexpr int M2 = Sh::M2, M3 = Sh::M3, NN = Sh::NN, NT = Sh::NT;
     static_assert(NN <= WIDE_NT && NT <= 64, "a node per thread, a direction's lines per wavefront");
+    static_assert(L::DOUBLES >= 3 * CFL_NT, "the CFL reduction runs in the operator's LDS");
     constexpr int V = NVars<EQ>::V;
     constexpr bool COMPACT = L::COMPACT;
     double* s_p64 = lds + L::RAW_DOUBLES;
@@ -294,7 +295,7 @@ __device__ __forceinline__ void stage_block_wide(const StageArgs<M, Real>& a, co
                 double* su[V];
 #pragma unroll
                 for (int h = 0; h < V; ++h) su[h] = s_u64[h];
-                if (!repair_element<EQ, M>(a.ph64, a.rk.w64, su, tid * M3)) atomicOr(a.status, 1);
+                if (!repair_element<EQ, M>(a.ph64, a.rk.w64, su, tid * M3)) *(volatile int*)a.status = 1;
             }
             __syncthreads();
             if (own)
@@ -317,44 +318,11 @@ __device__ __forceinline__ void stage_block_wide(const StageArgs<M, Real>& a, co
     }
 
     // ---- CFL partials of the new state (last stage of a step) -------------
-    // Maxima over the element's nodes as LDS maxima of the bit patterns (all
-    // values are >= 0; a NaN counts as 0, as in block_cfl's comparisons).
     if (a.cfl_part) {
-        if (own) {
-            unsigned long long* m = s_max + 4 * (tid / M3);
-            auto put = [&](int k, double x) {
-                if (x > 0.0) atomicMax(&m[k], (unsigned long long)__double_as_longlong(x));
-            };
-            put(0, lambda_max64<EQ, 0>(a.ph64, st));
-            put(1, lambda_max64<EQ, 1>(a.ph64, st));
-            put(2, lambda_max64<EQ, 2>(a.ph64, st));
-            const double v0 = fabs(st[1] / st[0]), v1 = fabs(st[2] / st[0]), v2 = fabs(st[3] / st[0]);
-            double v = v0 > v1 ? v0 : v1;
-            v = v > v2 ? v : v2;
-            put(3, v);
-        }
-        __syncthreads();
-        if (tid == 0) {
-            double dtb = 1.7976931348623157e308, lmb = 0.0, vmb = 0.0;
-            for (int k = 0; k < BE && e0 + k < a.nelem; ++k) {
-                const long long e = e0 + k;
-                const double m0 = __longlong_as_double((long long)s_max[4 * k + 0]);
-                const double m1 = __longlong_as_double((long long)s_max[4 * k + 1]);
-                const double m2 = __longlong_as_double((long long)s_max[4 * k + 2]);
-                const double vm = __longlong_as_double((long long)s_max[4 * k + 3]);
-                const double t0 = a.delta[e * 3 + 0] / m0, t1 = a.delta[e * 3 + 1] / m1, t2 = a.delta[e * 3 + 2] / m2;
-                double dte = t0 < t1 ? t0 : t1;
-                dte = dte < t2 ? dte : t2;
-                double lme = m0 > m1 ? m0 : m1;
-                lme = lme > m2 ? lme : m2;
-                dtb = dte < dtb ? dte : dtb;
-                lmb = lme > lmb ? lme : lmb;
-                vmb = vm > vmb ? vm : vmb;
-            }
-            double* out = a.cfl_part + 4 * blk;
-            out[0] = dtb;
-            out[1] = lmb;
-            out[2] = vmb;
+        block_cfl_nodes<EQ, M, BE>(a.ph64, a.delta, e0, a.nelem, own, st, s_max, a.cfl_part + 4 * blk);
+        if (a.fin.ticket) {
+            __syncthreads();  // the operator's LDS is free
+            cfl_last_block(a.cfl_part, int(gridDim.x), a.fin, M, reinterpret_cast<double (*)[CFL_NT]>(lds), s_bad);
         }
     }
 }

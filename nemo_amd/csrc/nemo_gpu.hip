@@ -127,38 +127,50 @@ long long nblocks_for(const Solver& s) {
 }
 
 template <int M>
-void launch_cfl_m(Solver& s) {
+void launch_cfl_m(Solver& s, const nemo::CflFinal& fin) {
     constexpr int BE = Tile<M>::BE;
     const nemo::Phys64 P = make_phys64(s.cfg);
+    const dim3 grid{unsigned(stage_blocks<M>(s))}, block{nemo::CFL_NT};
     if (s.cfg.equations == NEMO_EQ_GLM_MHD)
-        hipLaunchKernelGGL((nemo::cfl_kernel<nemo::EQ_MHD, M, BE>), dim3(unsigned(stage_blocks<M>(s))),
-                           dim3(BE * M * M), 0, s.stream, s.u[s.cur], s.delta, s.nelem, P, s.part);
+        hipLaunchKernelGGL((nemo::cfl_kernel<nemo::EQ_MHD, M, BE>), grid, block, 0, s.stream, s.u[s.cur], s.delta,
+                           s.nelem, P, s.part, fin);
     else
-        hipLaunchKernelGGL((nemo::cfl_kernel<nemo::EQ_EULER, M, BE>), dim3(unsigned(stage_blocks<M>(s))),
-                           dim3(BE * M * M), 0, s.stream, s.u[s.cur], s.delta, s.nelem, P, s.part);
+        hipLaunchKernelGGL((nemo::cfl_kernel<nemo::EQ_EULER, M, BE>), grid, block, 0, s.stream, s.u[s.cur], s.delta,
+                           s.nelem, P, s.part, fin);
 }
 
-int launch_finalize(Solver& s, long long hist_slot) {
+// Where a CFL reduction's result goes (hist_slot < 0: not into the history).
+nemo::CflFinal cfl_final(const Solver& s, long long hist_slot, double* host = nullptr) {
+    return nemo::CflFinal{s.dt_dev, hist_slot >= 0 ? s.hist : nullptr, hist_slot, host, s.cfl_ticket, s.cfg.cfl};
+}
+
+int launch_finalize(Solver& s, const nemo::CflFinal& fin) {
     const long long npart = nblocks_for(s);
     long long G = (npart + nemo::CFL_NT - 1) / nemo::CFL_NT;
     G = G < 1 ? 1 : (G > nemo::CFL_GRID ? nemo::CFL_GRID : G);
-    hipLaunchKernelGGL(nemo::cfl_finalize, dim3(unsigned(G)), dim3(nemo::CFL_NT), 0, s.stream, s.part, npart,
-                       s.cfg.cfl, s.M, s.dt_dev, hist_slot >= 0 ? s.hist : nullptr, hist_slot, s.cfl_red,
-                       s.cfl_ticket);
+    hipLaunchKernelGGL(nemo::cfl_finalize, dim3(unsigned(G)), dim3(nemo::CFL_NT), 0, s.stream, s.part, npart, s.M, fin,
+                       s.cfl_red);
     HIP_TRY(hipGetLastError());
     return NEMO_OK;
 }
 
-// CFL time step of the current state into dt_dev (and hist[hist_slot]).
-int launch_cfl(Solver& s, long long hist_slot) {
+// CFL time step of the current state into dt_dev (and hist, host).
+int launch_cfl(Solver& s, const nemo::CflFinal& fin) {
+    const bool fused = nblocks_for(s) <= nemo::CFL_FUSE;
+    nemo::CflFinal in = fin;
+    if (!fused) in.ticket = nullptr;
     switch (s.M) {
-    case 3: launch_cfl_m<3>(s); break;
-    case 4: launch_cfl_m<4>(s); break;
-    case 5: launch_cfl_m<5>(s); break;
+    case 3: launch_cfl_m<3>(s, in); break;
+    case 4: launch_cfl_m<4>(s, in); break;
+    case 5: launch_cfl_m<5>(s, in); break;
     default: return fail(NEMO_ERR_ARG, "n_poly must be 2, 3 or 4");
     }
     HIP_TRY(hipGetLastError());
-    return launch_finalize(s, hist_slot);
+    return fused ? NEMO_OK : launch_finalize(s, fin);
+}
+
+bool stage_takes_wide(const Solver& s, const LaunchOpts& o) {
+    return s.M == 3 ? takes_wide<3>(s, o) : (s.M == 4 ? takes_wide<4>(s, o) : takes_wide<5>(s, o));
 }
 
 int check_ready(Solver* s) {
@@ -168,13 +180,12 @@ int check_ready(Solver* s) {
     return NEMO_OK;
 }
 
+// Waits for the stream and turns the kernels' repair flag into an error.
 int status_check(Solver* s) {
-    int code = 0;
-    HIP_TRY(hipMemcpyAsync(&code, s->status, sizeof(int), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (code) {
-        HIP_TRY(hipMemsetAsync(s->status, 0, sizeof(int), s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
+    volatile int* flag = s->status;
+    if (*flag) {
+        *flag = 0;
         return fail(NEMO_ERR_STATE, "positivity repair failed (kernel_repair returned false)");
     }
     return NEMO_OK;
@@ -292,7 +303,6 @@ int set_mesh(Solver& s, int64_t nelem, const int32_t* nbr, const double* delta, 
         if (s.nslots > 0)
             HIP_TRY(hipMalloc(&s.mortar_flux, size_t(s.nslots) * size_t(s.V) * size_t(s.M * s.M) * sizeof(double)));
     }
-    if (!s.counter) HIP_TRY(hipMalloc(&s.counter, sizeof(int)));
     HIP_TRY(hipMemcpyAsync(s.nbr, nbr, size_t(nelem) * 6 * sizeof(int32_t), hipMemcpyHostToDevice, s.stream));
     HIP_TRY(hipMemcpyAsync(s.delta, delta, size_t(nelem) * 3 * sizeof(double), hipMemcpyHostToDevice, s.stream));
     if (nmortar > 0)
@@ -409,28 +419,42 @@ int nemo_gpu_create(const nemo_gpu_config* cfg, void** handle) {
         return fail(NEMO_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
     }
     staging_retain();
-    if (hipMalloc(&s->dt_dev, 8 * sizeof(double)) != hipSuccess ||
-        hipMalloc(&s->mlp_p, nemo::MLP_NP * sizeof(float)) != hipSuccess ||
-        hipMalloc(&s->mlp_inf, nemo::MLP_NP * sizeof(float)) != hipSuccess ||
-        hipMalloc(&s->mlp_m, nemo::MLP_NP * sizeof(float)) != hipSuccess ||
-        hipMalloc(&s->mlp_v, nemo::MLP_NP * sizeof(float)) != hipSuccess ||
-        hipMalloc(&s->mlp_stats, 3 * sizeof(unsigned long long)) != hipSuccess ||
-        hipMalloc(&s->status, sizeof(int)) != hipSuccess ||
-        hipMalloc(&s->cfl_red, 3 * nemo::CFL_GRID * sizeof(double)) != hipSuccess ||
-        hipMalloc(&s->cfl_ticket, sizeof(unsigned int)) != hipSuccess) {
+    // one zeroed device allocation for the handle's small buffers, one pinned
+    // page for what the kernels report
+    size_t used = 0;
+    auto part = [&](size_t bytes) {
+        const size_t at = used;
+        used += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    const size_t at_dt = part(8 * sizeof(double)), at_stats = part(3 * sizeof(unsigned long long)),
+                 at_ticket = part(sizeof(unsigned int)), at_counter = part(sizeof(int)),
+                 at_red = part(3 * nemo::CFL_GRID * sizeof(double)), at_p = part(nemo::MLP_NP * sizeof(float)),
+                 at_inf = part(nemo::MLP_NP * sizeof(float)), at_m = part(nemo::MLP_NP * sizeof(float)),
+                 at_v = part(nemo::MLP_NP * sizeof(float));
+    if (hipMalloc(&s->small, used) != hipSuccess || hipMemset(s->small, 0, used) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&s->host), 4 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
         nemo_gpu_destroy(s);  // frees whichever of them were allocated
         return fail(NEMO_ERR_HIP, "hipMalloc failed");
     }
+    char* const base = static_cast<char*>(s->small);
+    s->dt_dev = reinterpret_cast<double*>(base + at_dt);
+    s->mlp_stats = reinterpret_cast<unsigned long long*>(base + at_stats);
+    s->cfl_ticket = reinterpret_cast<unsigned int*>(base + at_ticket);
+    s->counter = reinterpret_cast<int*>(base + at_counter);
+    s->cfl_red = reinterpret_cast<double*>(base + at_red);
+    s->mlp_p = reinterpret_cast<float*>(base + at_p);
+    s->mlp_inf = reinterpret_cast<float*>(base + at_inf);
+    s->mlp_m = reinterpret_cast<float*>(base + at_m);
+    s->mlp_v = reinterpret_cast<float*>(base + at_v);
     // this device's copy of the allocation-free analysis scratch
     if (hipError_t e = scratch_device_ptr(&s->scratch); e != hipSuccess) {
         s->scratch = nullptr;
         nemo_gpu_destroy(s);
         return fail(NEMO_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
     }
-    (void)hipMemset(s->status, 0, sizeof(int));
-    (void)hipMemset(s->cfl_ticket, 0, sizeof(unsigned int));
-    (void)hipMemset(s->dt_dev, 0, 8 * sizeof(double));
-    (void)hipMemset(s->mlp_stats, 0, 3 * sizeof(unsigned long long));
+    s->status = reinterpret_cast<int*>(s->host + 3);
+    *s->status = 0;
     *handle = s;
     return NEMO_OK;
 }
@@ -440,20 +464,12 @@ int nemo_gpu_destroy(void* handle) {
     if (!s) return NEMO_OK;
     (void)hipStreamSynchronize(s->stream);
     free_mesh_buffers(*s);
-    (void)hipFree(s->dt_dev);
-    (void)hipFree(s->status);
-    (void)hipFree(s->counter);
+    (void)hipFree(s->small);
+    (void)hipHostFree(s->host);
     (void)hipFree(s->units);
     (void)hipFree(s->an_part);
     (void)hipFree(s->an_out);
-    (void)hipFree(s->mlp_p);
-    (void)hipFree(s->mlp_inf);
-    (void)hipFree(s->mlp_m);
-    (void)hipFree(s->mlp_v);
-    (void)hipFree(s->mlp_stats);
     (void)hipFree(s->hist);
-    (void)hipFree(s->cfl_red);
-    (void)hipFree(s->cfl_ticket);
     for (auto& p : s->ev) {
         (void)hipEventDestroy(p.first);
         (void)hipEventDestroy(p.second);
@@ -653,10 +669,9 @@ int nemo_gpu_analyze_noalloc(void* handle, double* sums_dev) {
 int nemo_gpu_calc_timestep(void* handle, double* dt, double* lmax, double* vmax) {
     Solver* s = static_cast<Solver*>(handle);
     if (int rc = check_ready(s)) return rc;
-    if (int rc = launch_cfl(*s, -1)) return rc;
-    double h[3];
-    HIP_TRY(hipMemcpyAsync(h, s->dt_dev, 3 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    if (int rc = launch_cfl(*s, cfl_final(*s, -1, s->host))) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
+    const volatile double* h = s->host;
     if (dt) *dt = h[0];
     if (lmax) *lmax = h[1];
     if (vmax) *vmax = h[2];
@@ -715,40 +730,38 @@ int nemo_gpu_run(void* handle, int32_t nsteps, double* dt_hist) {
     // The first step's dt comes from a standalone reduction; every later dt
     // from the CFL partials that the last stage of the previous step writes.
     if (nsteps > 0)
-        if (int rc = launch_cfl(*s, dt_hist ? 0 : -1)) return rc;
+        if (int rc = launch_cfl(*s, cfl_final(*s, dt_hist ? 0 : -1))) return rc;
+    const bool fused = nblocks_for(*s) <= nemo::CFL_FUSE && stage_takes_wide(*s, LaunchOpts());
     for (int it = 0; it < nsteps; ++it) {
         const bool more = it + 1 < nsteps;
         for (int st = 1; st <= 5; ++st) {
             double* part = (st == 5 && more) ? s->part : nullptr;
             LaunchOpts o;
             o.refresh = st == 1;
+            if (part && fused) o.fin = cfl_final(*s, dt_hist ? it + 1 : -1);
             if (int rc = launch_stage(*s, st, 0.0, s->dt_dev, nullptr, nullptr, part, o)) return rc;
             if (st == 1) ++s->step_counter;
             s->cur ^= 1;
         }
-        if (more)
-            if (int rc = launch_finalize(*s, dt_hist ? it + 1 : -1)) return rc;
+        if (more && !fused)
+            if (int rc = launch_finalize(*s, cfl_final(*s, dt_hist ? it + 1 : -1))) return rc;
     }
     if (dt_hist && nsteps > 0)
         HIP_TRY(hipMemcpyAsync(dt_hist, s->hist, size_t(nsteps) * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
     return status_check(s);
 }
 
 int nemo_gpu_synchronize(void* handle) {
     Solver* s = static_cast<Solver*>(handle);
     if (!s) return fail(NEMO_ERR_ARG, "null handle");
-    HIP_TRY(hipStreamSynchronize(s->stream));
     return status_check(s);
 }
 
 int nemo_gpu_get_status(void* handle, int32_t* code) {
     Solver* s = static_cast<Solver*>(handle);
     if (!s || !code) return fail(NEMO_ERR_ARG, "null argument");
-    int c = 0;
-    HIP_TRY(hipMemcpyAsync(&c, s->status, sizeof(int), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    *code = c;
+    *code = *(volatile int*)s->status;
     return NEMO_OK;
 }
 

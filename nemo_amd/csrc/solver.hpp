@@ -37,28 +37,30 @@ struct Solver {
     int32_t* bfaces = nullptr;         // [nbound][3]: element, face, kind
     long long nslots = 0;              // 5*nmortar + nbound face slots
     double* mortar_flux = nullptr;     // [nslots][V][M*M]: mortar slots, then boundary slots
-    int* counter = nullptr;            // remap fallbacks
+    void* small = nullptr;             // one allocation: the pointers marked (s)
+    int* counter = nullptr;            // (s) remap fallbacks
     int32_t* units = nullptr;          // replacement units of the last remesh
     long long units_cap = 0;
     double* an_part = nullptr;         // analysis partials
     long long an_cap = 0;
     double* an_out = nullptr;          // [NEMO_ANALYZE_NSUMS]
-    double* scratch = nullptr;
-    double* cfl_red = nullptr;         // [3 * CFL_GRID] second level of the CFL reduction
-    unsigned int* cfl_ticket = nullptr;  // blocks done in the current CFL reduction         // this device's `scratch` (allocation-free analysis)
-    double* dt_dev = nullptr;  // [8]: dt, lmax, vmax, glm c_h, glm alpha
+    double* scratch = nullptr;         // this device's `scratch` (allocation-free analysis)
+    double* cfl_red = nullptr;         // (s) [3 * CFL_GRID] second level of the CFL reduction
+    unsigned int* cfl_ticket = nullptr;  // (s) blocks done in the current CFL reduction
+    double* dt_dev = nullptr;  // (s) [8]: dt, lmax, vmax, glm c_h, glm alpha
     double* part = nullptr;    // per-block CFL partials [nblocks][4]
-    int* status = nullptr;
+    double* host = nullptr;    // pinned: dt, lmax, vmax of the last reduction that asked for them
+    int* status = nullptr;     // pinned, written by the stage kernels: a repair failed
     double* hist = nullptr;
     long long hist_cap = 0;
     hipStream_t stream = nullptr;
 
     // learned indicator
-    float* mlp_p = nullptr;     // canonical parameters
-    float* mlp_inf = nullptr;   // inference layout
-    float* mlp_m = nullptr;     // Adam moments
-    float* mlp_v = nullptr;
-    unsigned long long* mlp_stats = nullptr;  // judged, overridden, fallback
+    float* mlp_p = nullptr;     // (s) canonical parameters
+    float* mlp_inf = nullptr;   // (s) inference layout
+    float* mlp_m = nullptr;     // (s) Adam moments
+    float* mlp_v = nullptr;     // (s)
+    unsigned long long* mlp_stats = nullptr;  // (s) judged, overridden, fallback
     double* alpha_step = nullptr;  // [nelem]
     bool mlp_ready = false;
     uint32_t step_counter = 0;
@@ -75,8 +77,14 @@ struct Solver {
 struct LaunchOpts {
     int refresh = 1;            // learned indicator: compute the factor of the step
     float* feat_out = nullptr;  // training data: features of every element
+    nemo::CflFinal fin{};       // with CFL partials: where the time step goes (ticket null: reduced apart)
     int alpha_only = 0;         // indicator only (Euler): the factor to alpha_out, no operator
 };
+
+// Whether the stage launch with these options takes the small-mesh form, whose
+// last block can reduce the CFL partials (defined in stage_launch.hpp).
+template <int M>
+bool takes_wide(const Solver& s, const LaunchOpts& o);
 
 // Stage launch of one polynomial degree (M = n_poly + 1 nodes per direction),
 // defined in stage_launch.hpp and instantiated in stage_m<M>.hip.

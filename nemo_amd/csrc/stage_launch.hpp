@@ -37,6 +37,7 @@ nemo::StageArgs<M, Real> make_args(Solver& s, int stage, double dt, const double
     a.glm = s.dt_dev + 3;
     a.status = s.status;
     a.cfl_part = cfl_part;
+    a.fin = o.fin;
     a.nelem = s.nelem;
     a.dt = dt;
     a.stage = stage;
@@ -161,6 +162,12 @@ long long wide_blocks(const nemo_gpu_config& c) {
     return M == 3 ? 2048 : 1536;
 }
 
+template <int M>
+bool takes_wide(const Solver& s, const LaunchOpts& o) {
+    const long long limit = s.cfg.precision == 1 ? wide_blocks<M, float>(s.cfg) : wide_blocks<M, double>(s.cfg);
+    return (s.nelem + Tile<M>::BE - 1) / Tile<M>::BE <= limit && !o.alpha_only && !o.feat_out;
+}
+
 template <int M, typename Real>
 int launch_stage_mr(Solver& s, int stage, double dt, const double* dt_dev, double* rhs_out, double* alpha_out,
                     double* cfl_part, const LaunchOpts& o) {
@@ -168,7 +175,7 @@ int launch_stage_mr(Solver& s, int stage, double dt, const double* dt_dev, doubl
     const int vol = s.cfg.volume, surf = s.cfg.surface;
     if (s.nmortar > 0 && !o.alpha_only) launch_mortar<M, Real>(s);
     if (s.nbound > 0 && !o.alpha_only) launch_boundary<M>(s);
-    if ((s.nelem + Tile<M>::BE - 1) / Tile<M>::BE <= wide_blocks<M, Real>(s.cfg) && !o.alpha_only && !o.feat_out)
+    if (takes_wide<M>(s, o))
         return launch_wide<M, Real>(s, a, o.refresh || rhs_out);
     if constexpr (M == 4) {
         // learned indicator, and the training-data pass of any Euler scheme

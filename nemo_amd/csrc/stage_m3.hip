@@ -2,6 +2,7 @@
 #include "stage_launch.hpp"
 
 namespace nemo_host {
+template bool takes_wide<3>(const Solver& s, const LaunchOpts& o);
 template int launch_stage_m<3>(Solver& s, int stage, double dt, const double* dt_dev, double* rhs_out,
                                 double* alpha_out, double* cfl_part, const LaunchOpts& o);
 }  // namespace nemo_host

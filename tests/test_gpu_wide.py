@@ -63,6 +63,36 @@ def test_euler_same_bits(N, prec, vol, surf, td, ind):
         assert np.array_equal(b.get_state(), s.get_state()[src])
 
 
+@pytest.mark.parametrize("N", [2, 3, 4])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_walls_and_open_sides(N, prec):
+    """Boundary faces, whose fluxes both forms take from a launch before them:
+    walls across y, open sides across z."""
+    limit, tile = {2: (2048, 7), 3: (6144, 4), 4: (1536, 2)}[N]
+    reps = limit * tile // int(np.prod(SMALL)) + 1
+    small, big, src = _tiled(SMALL, reps)
+    kinds = [None, None, meshmod.BC_SLIP_WALL, meshmod.BC_SLIP_WALL, meshmod.BC_TRANSMISSIVE, meshmod.BC_TRANSMISSIVE]
+    cfg = solver.make_config(N=N, volume=_lib.VOL_EC, surface=_lib.SURF_HLLC, indicator=_lib.IND_PP, repair=1,
+                             timedisc=_lib.TD_LSRK54, precision=prec)
+    rng = np.random.default_rng(N)
+    u = np.zeros((small.nelem, 5, (N + 1) ** 3))
+    u[:, 0] = 1.0 + 0.2 * rng.random(u[:, 0].shape)
+    u[:, 1:4] = 0.3 * rng.standard_normal(u[:, 1:4].shape)
+    u[:, 4] = 2.5 + 0.5 * (u[:, 1:4] ** 2).sum(1)
+    print(f"forms walls N={N} precision={prec} elements={len(src)}", flush=True)
+    out = []
+    for m, v in ((small, u), (big, u[src])):
+        with solver.Solver(cfg) as s:
+            s.upload_mesh(meshmod.with_boundaries(m, kinds))
+            s.set_state(v)
+            out.append(s.kernel_calc_flux())
+    # the faces' fluxes are FP64 in both, to rounding (1e-12 and, through the
+    # FP32 operator, 1e-5 of the largest value: the bounds of the boundary tests)
+    tol = 1e-5 if prec else 1e-12
+    for h in range(5):
+        assert np.abs(out[1][:, h] - out[0][src][:, h]).max() <= tol * np.abs(out[1][:, h]).max(), h
+
+
 @pytest.mark.parametrize("N,surf", [(2, _lib.SURF_HLLD), (3, _lib.SURF_HLLD), (3, _lib.SURF_RUSANOV),
                                     (4, _lib.SURF_RUSANOV)])
 @pytest.mark.parametrize("prec", [0, 1])
