@@ -20,7 +20,9 @@
 
 #include "host_ops.hpp"
 #include "dg_batch.hpp"
+#include "dg_stage_wide.hpp"
 #include "transfer.hpp"
+#include "wide_rule.hpp"
 
 namespace {
 
@@ -144,6 +146,14 @@ template <int M, typename Real>
 void launch_group_stage(Batch* b, Group& gr, int stage, bool cfl) {
     constexpr int BE = Tile<M>::BE;
     const auto a = batch_args<M, Real>(b, gr, stage, cfl);
+    if (b->grid_per_cu == 0 && gr.nblocks <= wide_blocks<M, Real>(b->cfg)) {
+        // few blocks: each on four wavefronts, with the same bits (4 runs of 5
+        // to 9 elements a side, FP64: 102 -> 59 us per stage of all degrees; 8
+        // runs of 6 to 12, FP32: 88 -> 60)
+        hipLaunchKernelGGL((nemo::stage_kernel_wide<nemo::EQ_EULER, M, BE, nemo::VOL_EC, nemo::SURF_HLLC, Real>),
+                           dim3(unsigned(gr.nblocks)), dim3(nemo::WIDE_NT), 0, b->stream, a);
+        return;
+    }
     if (b->grid_per_cu == 0) {
         // one workgroup per block: the plain stage kernel (its blocks are
         // dealt to the XCDs in contiguous stretches).  The persistent loop

@@ -252,7 +252,7 @@ __device__ __forceinline__ void stage_block_wide(const StageArgs<M, Real>& a, co
             for (int h = 0; h < V; ++h) a.rhs_out[h * EM3 + gi0] = f[h];
         return;
     }
-    const double dt = a.dt_dev ? *a.dt_dev : a.dt;
+    const double dt = a.dt_run ? a.dt_run[a.block_run[blk]] : (a.dt_dev ? *a.dt_dev : a.dt);
     double st[V];
     if (own) {
 #pragma unroll
