@@ -419,8 +419,8 @@ int nemo_gpu_create(const nemo_gpu_config* cfg, void** handle) {
         return fail(NEMO_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
     }
     staging_retain();
-    // one zeroed device allocation for the handle's small buffers, one pinned
-    // page for what the kernels report
+    // one zeroed device allocation for the handle's small buffers, and pinned
+    // memory for what the kernels report
     size_t used = 0;
     auto part = [&](size_t bytes) {
         const size_t at = used;
@@ -432,8 +432,8 @@ int nemo_gpu_create(const nemo_gpu_config* cfg, void** handle) {
                  at_red = part(3 * nemo::CFL_GRID * sizeof(double)), at_p = part(nemo::MLP_NP * sizeof(float)),
                  at_inf = part(nemo::MLP_NP * sizeof(float)), at_m = part(nemo::MLP_NP * sizeof(float)),
                  at_v = part(nemo::MLP_NP * sizeof(float));
-    if (hipMalloc(&s->small, used) != hipSuccess || hipMemset(s->small, 0, used) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&s->host), 4 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    s->host = static_cast<double*>(report_get());
+    if (!s->host || hipMalloc(&s->small, used) != hipSuccess || hipMemset(s->small, 0, used) != hipSuccess) {
         nemo_gpu_destroy(s);  // frees whichever of them were allocated
         return fail(NEMO_ERR_HIP, "hipMalloc failed");
     }
@@ -465,7 +465,7 @@ int nemo_gpu_destroy(void* handle) {
     (void)hipStreamSynchronize(s->stream);
     free_mesh_buffers(*s);
     (void)hipFree(s->small);
-    (void)hipHostFree(s->host);
+    report_put(s->host);
     (void)hipFree(s->units);
     (void)hipFree(s->an_part);
     (void)hipFree(s->an_out);

@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <cstdint>
 #include <cstring>
 #include <mutex>
 #include <new>
@@ -267,6 +268,40 @@ bool staged_copy(hipStream_t stream, double* dev, double* host, size_t bytes, bo
 }  // namespace
 
 namespace nemo_host {
+
+// The reports of up to 64 handles share one pinned page, which stays until the
+// process ends: a pinned allocation takes longer than the rest of a handle's
+// creation.  Further handles allocate their own.
+namespace {
+constexpr size_t REPORT_BYTES = 64, REPORT_SLOTS = 64;
+std::mutex report_mu;
+char* report_page = nullptr;
+uint64_t report_used = 0;
+}  // namespace
+
+void* report_get() {
+    std::lock_guard<std::mutex> lock(report_mu);
+    if (!report_page && hipHostMalloc(reinterpret_cast<void**>(&report_page), REPORT_BYTES * REPORT_SLOTS,
+                                      hipHostMallocPortable) != hipSuccess)
+        report_page = nullptr;
+    if (report_page && ~report_used) {
+        const int k = __builtin_ctzll(~report_used);
+        report_used |= uint64_t(1) << k;
+        return report_page + REPORT_BYTES * size_t(k);
+    }
+    void* p = nullptr;
+    return hipHostMalloc(&p, REPORT_BYTES, hipHostMallocPortable) == hipSuccess ? p : nullptr;
+}
+
+void report_put(void* p) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lock(report_mu);
+    const size_t at = size_t(static_cast<char*>(p) - report_page);
+    if (report_page && static_cast<char*>(p) >= report_page && at < REPORT_BYTES * REPORT_SLOTS)
+        report_used &= ~(uint64_t(1) << (at / REPORT_BYTES));
+    else
+        (void)hipHostFree(p);
+}
 
 void staging_retain() {
     std::lock_guard<std::mutex> lock(refs_mu);

@@ -23,4 +23,9 @@ hipError_t state_to_device(hipStream_t stream, const double* host, double* scrat
 void staging_retain();
 void staging_release();
 
+// 64 bytes of pinned host memory that kernels write their reports to; nullptr
+// if there is none to be had.
+void* report_get();
+void report_put(void* p);
+
 }  // namespace nemo_host
