@@ -10,8 +10,8 @@
 // blending factor meanwhile, and the 256 threads own one node each for the
 // loads, the Runge-Kutta update, the positivity check and the CFL partials.
 // The terms are added to the node accumulators in the order of stage_kernel,
-// a barrier apart, with the same operations, so both kernels return the same
-// bits and a mesh may be large enough for one or the other.
+// a barrier apart, with the same operations: Euler results have the same bits
+// in both forms; GLM-MHD sums rotated states and agrees to rounding.
 #pragma once
 
 #include "dg_stage.hpp"
