@@ -519,7 +519,9 @@ int nemo_gpu_batch_create(const nemo_gpu_config* cfg, int32_t nruns, const int32
         bool ok = hipMemcpy(gr.nbr, nbr.data(), nbr.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess &&
                   hipMemcpy(gr.delta, delta.data(), delta.size() * sizeof(double), hipMemcpyHostToDevice) == hipSuccess &&
                   hipMemcpy(gr.block_run, brun.data(), brun.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess &&
-                  hipMemset(gr.r0, 0, sb) == hipSuccess && hipMemset(gr.r1, 0, sb) == hipSuccess;
+                  // (on the batch's stream, which does not wait for the null stream)
+                  hipMemsetAsync(gr.r0, 0, sb, b->stream) == hipSuccess &&
+                  hipMemsetAsync(gr.r1, 0, sb, b->stream) == hipSuccess;
         const double vals[5] = {1.0, 0.0, 0.0, 0.0, 1.0 / (cfg->gamma - 1.0)};
         for (int v = 0; v < 5 && ok; ++v) {
             std::fill(ghost.begin(), ghost.end(), vals[v]);
@@ -541,7 +543,8 @@ int nemo_gpu_batch_create(const nemo_gpu_config* cfg, int32_t nruns, const int32
         hipMemcpy(b->run_pstart, pstart.data(), size_t(nruns) * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->run_pcount, pcount.data(), size_t(nruns) * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->run_M_dev, rm.data(), size_t(nruns) * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(b->status, 0, sizeof(int)) != hipSuccess || hipMemset(b->step_ctr, 0, sizeof(unsigned long long)) != hipSuccess)
+        hipMemsetAsync(b->status, 0, sizeof(int), b->stream) != hipSuccess ||
+        hipMemsetAsync(b->step_ctr, 0, sizeof(unsigned long long), b->stream) != hipSuccess)
         return bail("hipMalloc of the batch tables failed");
     *handle = b;
     return NEMO_OK;

@@ -420,7 +420,8 @@ int nemo_gpu_create(const nemo_gpu_config* cfg, void** handle) {
     }
     staging_retain();
     // one zeroed device allocation for the handle's small buffers, and pinned
-    // memory for what the kernels report
+    // memory for what the kernels report; zeroed on the handle's own stream,
+    // which does not wait for the null stream
     size_t used = 0;
     auto part = [&](size_t bytes) {
         const size_t at = used;
@@ -433,7 +434,8 @@ int nemo_gpu_create(const nemo_gpu_config* cfg, void** handle) {
                  at_inf = part(nemo::MLP_NP * sizeof(float)), at_m = part(nemo::MLP_NP * sizeof(float)),
                  at_v = part(nemo::MLP_NP * sizeof(float));
     s->host = static_cast<double*>(report_get());
-    if (!s->host || hipMalloc(&s->small, used) != hipSuccess || hipMemset(s->small, 0, used) != hipSuccess) {
+    if (!s->host || hipMalloc(&s->small, used) != hipSuccess ||
+        hipMemsetAsync(s->small, 0, used, s->stream) != hipSuccess) {
         nemo_gpu_destroy(s);  // frees whichever of them were allocated
         return fail(NEMO_ERR_HIP, "hipMalloc failed");
     }
