@@ -209,6 +209,19 @@ int nemo_gpu_run(void *handle, int32_t nsteps, double *dt_hist);
 int nemo_gpu_synchronize(void *handle);
 int nemo_gpu_get_status(void *handle, int32_t *code);
 
+/* Form of the stage kernel, for measurements and tests: NEMO_FORM_AUTO
+ * (default) takes the faster one for the mesh's number of blocks of elements,
+ * NEMO_FORM_ONE_WAVE runs a block on one wavefront, NEMO_FORM_FOUR_WAVES on
+ * four.  Euler results have the same bits in both (the learned indicator's
+ * network: to FP32 rounding), GLM-MHD results agree to rounding.
+ * Indicator-only launches of the Euler equations and
+ * nemo_gpu_indicator_features run on one wavefront in any case; GLM-MHD with
+ * HLLD at n_poly = 4 is built for four, NEMO_FORM_ONE_WAVE is refused there. */
+#define NEMO_FORM_AUTO 0
+#define NEMO_FORM_ONE_WAVE 1
+#define NEMO_FORM_FOUR_WAVES 2
+int nemo_gpu_set_form(void *handle, int32_t form);
+
 /* Kernel timing with HIP events on the solver's stream: enable, then read
  * the number of stage launches and their summed duration in milliseconds
  * (reading synchronises and resets the counters). */
@@ -282,6 +295,10 @@ int nemo_gpu_batch_run(void *handle, int32_t nsteps, int32_t use_graph, double *
  * block of elements) and the XCD-contiguous block map on or off.  Default:
  * one launch per stage, one workgroup per block, order 0. */
 int nemo_gpu_batch_set_launch(void *handle, int32_t grid_per_cu, int32_t xcd_map, int32_t one_launch, int32_t order);
+/* Form of the stage kernel as in nemo_gpu_set_form, where each degree has its
+ * own launch with one workgroup per block (one_launch = 0, grid_per_cu = 0);
+ * the other geometries run a block on one wavefront. */
+int nemo_gpu_batch_set_form(void *handle, int32_t form);
 /* Times `steps` steps of every candidate geometry on the current states
  * (which are restored afterwards), keeps the fastest and reports it. */
 int nemo_gpu_batch_autotune(void *handle, int32_t steps, int32_t *grid_per_cu, int32_t *xcd_map, int32_t *one_launch,

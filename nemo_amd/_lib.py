@@ -22,6 +22,7 @@ SURF_RUSANOV, SURF_HLLC, SURF_HLLD = 0, 1, 2
 IND_NONE, IND_PP, IND_MLP = 0, 1, 2
 MLP_NPARAMS = 8705
 TD_LSRK54, TD_SSPRK54 = 0, 1
+FORM_AUTO, FORM_ONE_WAVE, FORM_FOUR_WAVES = 0, 1, 2
 
 
 class Config(ctypes.Structure):
@@ -96,6 +97,8 @@ SIGNATURES = {
     "nemo_gpu_batch_set_launch": [_VP, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32],
     "nemo_gpu_batch_autotune": [_VP, ctypes.c_int32, _PI32, _PI32, _PI32, _PI32, _P],
     "nemo_gpu_batch_tune_table": [_VP, ctypes.c_int32, _PI32, _PI32, _P],
+    "nemo_gpu_batch_set_form": [_VP, ctypes.c_int32],
+    "nemo_gpu_set_form": [_VP, ctypes.c_int32],
     "nemo_gpu_set_timing": [_VP, ctypes.c_int32],
     "nemo_gpu_copy_calibration": [_VP, ctypes.c_int64],
     "nemo_gpu_check_arithmetic": [_VP, ctypes.c_int64, ctypes.c_uint64, ctypes.POINTER(ctypes.c_int64),

@@ -70,9 +70,10 @@ struct Batch {
     // degree groups in the one launch (0: M = 5, 4, 3, the costliest blocks
     // first; 1: M = 3, 4, 5)
     int grid_per_cu = 0, xcd = 1, one_launch = 1, order = 0;
+    int form = NEMO_FORM_AUTO;  // of the per-degree stage kernel
     hipGraphExec_t graph = nullptr;
     int graph_cur[3] = {-1, -1, -1};
-    int graph_grid = -1, graph_xcd = -1, graph_one = -1, graph_order = -1;
+    int graph_grid = -1, graph_xcd = -1, graph_one = -1, graph_order = -1, graph_form = -1;
     // stage arguments of the one launch for the ten stages of two steps
     // (slot k: stage k % 5 + 1 from buffer parity k & 1), device memory
     void* margs = nullptr;
@@ -154,7 +155,7 @@ template <int M, typename Real>
 void launch_group_stage(Batch* b, hipStream_t stream, Group& gr, int stage, bool cfl) {
     constexpr int BE = Tile<M>::BE;
     const auto a = batch_args<M, Real>(b, gr, stage, cfl);
-    if (b->grid_per_cu == 0 && gr.nblocks <= wide_blocks<M, Real>(b->cfg)) {
+    if (b->grid_per_cu == 0 && wide_form<M, Real>(b->cfg, b->form, gr.nblocks)) {
         // few blocks: each on four wavefronts, with the same bits (4 runs of 5
         // to 9 elements a side, FP64: 102 -> 59 us per stage of all degrees; 8
         // runs of 6 to 12, FP32: 88 -> 60)
@@ -373,7 +374,7 @@ int launch_cfl(Batch* b) {
 
 bool graph_matches(const Batch* b) {
     if (!b->graph || b->graph_grid != b->grid_per_cu || b->graph_xcd != b->xcd || b->graph_one != b->one_launch ||
-        b->graph_order != b->order)
+        b->graph_order != b->order || b->graph_form != b->form)
         return false;
     for (int i = 0; i < 3; ++i)
         if (b->g[i].nelem && b->graph_cur[i] != b->g[i].cur) return false;
@@ -408,6 +409,7 @@ int build_graph(Batch* b) {
     b->graph_xcd = b->xcd;
     b->graph_one = b->one_launch;
     b->graph_order = b->order;
+    b->graph_form = b->form;
     return NEMO_OK;
 }
 
@@ -601,6 +603,13 @@ int nemo_gpu_batch_set_launch(void* handle, int32_t grid_per_cu, int32_t xcd_map
     b->xcd = xcd_map ? 1 : 0;
     b->one_launch = one_launch ? 1 : 0;
     b->order = order;
+    return NEMO_OK;
+}
+
+int nemo_gpu_batch_set_form(void* handle, int32_t form) {
+    Batch* b = static_cast<Batch*>(handle);
+    if (!b || form < NEMO_FORM_AUTO || form > NEMO_FORM_FOUR_WAVES) return fail(NEMO_ERR_ARG, "invalid arguments");
+    b->form = form;
     return NEMO_OK;
 }
 

@@ -1060,6 +1060,17 @@ int nemo_gpu_check_arithmetic(void* handle, int64_t n, uint64_t seed, int64_t* d
     return NEMO_OK;
 }
 
+int nemo_gpu_set_form(void* handle, int32_t form) {
+    Solver* s = static_cast<Solver*>(handle);
+    if (!s) return fail(NEMO_ERR_ARG, "null handle");
+    if (form < NEMO_FORM_AUTO || form > NEMO_FORM_FOUR_WAVES) return fail(NEMO_ERR_ARG, "invalid form");
+    if (form == NEMO_FORM_ONE_WAVE && s->cfg.equations == NEMO_EQ_GLM_MHD && s->cfg.surface == NEMO_SURF_HLLD &&
+        s->M == 5)
+        return fail(NEMO_ERR_ARG, "GLM-MHD with HLLD at n_poly = 4 is built for four wavefronts per block");
+    s->form = form;
+    return NEMO_OK;
+}
+
 int nemo_gpu_set_timing(void* handle, int32_t enable) {
     Solver* s = static_cast<Solver*>(handle);
     if (!s) return fail(NEMO_ERR_ARG, "null handle");

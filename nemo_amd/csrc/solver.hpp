@@ -66,6 +66,7 @@ struct Solver {
     uint32_t step_counter = 0;
     double sample_fraction = 0.05, judge_tol = 0.05;
 
+    int form = NEMO_FORM_AUTO;  // of the stage kernel
     bool timing = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
     size_t ev_used = 0;

@@ -129,8 +129,10 @@ int launch_wide(Solver& s, const nemo::StageArgs<M, Real>& a, bool net);
 
 template <int M>
 bool takes_wide(const Solver& s, const LaunchOpts& o) {
-    const long long limit = s.cfg.precision == 1 ? wide_blocks<M, float>(s.cfg) : wide_blocks<M, double>(s.cfg);
-    return (s.nelem + Tile<M>::BE - 1) / Tile<M>::BE <= limit && !o.alpha_only && !o.feat_out;
+    const long long nblocks = (s.nelem + Tile<M>::BE - 1) / Tile<M>::BE;
+    const bool wide = s.cfg.precision == 1 ? wide_form<M, float>(s.cfg, s.form, nblocks)
+                                           : wide_form<M, double>(s.cfg, s.form, nblocks);
+    return wide && !o.alpha_only && !o.feat_out;
 }
 
 template <int M, typename Real>

@@ -45,4 +45,11 @@ long long wide_blocks(const nemo_gpu_config& c) {
     return M == 3 ? 2048 : 1536;
 }
 
+// Whether a launch over nblocks blocks takes the small-mesh form; `form` is
+// NEMO_FORM_AUTO or one of the two.
+template <int M, typename Real>
+bool wide_form(const nemo_gpu_config& c, int form, long long nblocks) {
+    return form == NEMO_FORM_AUTO ? nblocks <= wide_blocks<M, Real>(c) : form == NEMO_FORM_FOUR_WAVES;
+}
+
 }  // namespace nemo_host

@@ -267,6 +267,11 @@ class Solver:
     def synchronize(self) -> None:
         self._call("nemo_gpu_synchronize", self._h)
 
+    def set_form(self, form: int) -> None:
+        """Form of the stage kernel (FORM_*): by the mesh's size, or a block of
+        elements on one wavefront or on four (measurements and tests)."""
+        self._call("nemo_gpu_set_form", self._h, ctypes.c_int32(form))
+
     # -- timing ------------------------------------------------------------------
     def set_timing(self, enable: bool) -> None:
         self._call("nemo_gpu_set_timing", self._h, ctypes.c_int32(1 if enable else 0))
@@ -395,6 +400,11 @@ class Batch:
         workgroup per block), XCD map, order of the degree groups."""
         self._call("nemo_gpu_batch_set_launch", self._h, ctypes.c_int32(grid_per_cu), ctypes.c_int32(int(xcd_map)),
                    ctypes.c_int32(int(one_launch)), ctypes.c_int32(order))
+
+    def set_form(self, form: int) -> None:
+        """Form of the stage kernel (FORM_*) where each degree has its own
+        launch with one workgroup per block."""
+        self._call("nemo_gpu_batch_set_form", self._h, ctypes.c_int32(form))
 
     def autotune(self, steps: int = 2) -> dict:
         """Time every candidate launch geometry, keep the fastest; returns it
