@@ -89,9 +89,9 @@ __device__ __forceinline__ void load_face_nodes(const StageArgs<M, Real>& a, lon
 }
 
 // The two face Riemann fluxes of line `tid` in direction D from the nodes um
-// and up across its ends, and jac = 2 / dx.  In the FP32 operator with INBLK
-// a neighbour inside the block is read from LDS (load_face_nodes).
-template <int D, int M, int BE, int SURF, bool INBLK, typename Real, typename TU>
+// and up across its ends, and jac = 2 / dx.  In the FP32 operator a neighbour
+// inside the block is read from LDS (load_face_nodes).
+template <int D, int M, int BE, int SURF, typename Real, typename TU>
 __device__ __forceinline__ void surface_fluxes(const StageArgs<M, Real>& a, int tid, long long e0,
                                                const TU (*s_u)[BE * M * M * M], const double* s_p64,
                                                const ElemGeom& geo, const double (&um)[5], const double (&up)[5],
@@ -122,23 +122,21 @@ __device__ __forceinline__ void surface_fluxes(const StageArgs<M, Real>& a, int 
         S1.p64 = s_p64[n1];
         Nm.p64 = pressure(a.ph64.gas, um);
         Np.p64 = pressure(a.ph64.gas, up);
-        if constexpr (INBLK) {
-            // neighbours inside the block: their staged nodes in LDS
-            const long long em = geo.nbr[2 * D], ep = geo.nbr[2 * D + 1];
-            const bool im = valid && in_block(em, e0, a.nelem, BE);
-            const bool ip = valid && in_block(ep, e0, a.nelem, BE);
-            const int nm = bslot<M>((im ? int(em - e0) : 0) * M3, nidx<D, M>(M - 1, ta, tb));
-            const int np = bslot<M>((ip ? int(ep - e0) : 0) * M3, nidx<D, M>(0, ta, tb));
+        // neighbours inside the block: their staged nodes in LDS
+        const long long em = geo.nbr[2 * D], ep = geo.nbr[2 * D + 1];
+        const bool im = valid && in_block(em, e0, a.nelem, BE);
+        const bool ip = valid && in_block(ep, e0, a.nelem, BE);
+        const int nm = bslot<M>((im ? int(em - e0) : 0) * M3, nidx<D, M>(M - 1, ta, tb));
+        const int np = bslot<M>((ip ? int(ep - e0) : 0) * M3, nidx<D, M>(0, ta, tb));
 #pragma unroll
-            for (int h = 0; h < 5; ++h) {
-                const Real lm = Real(s_u[h][nm]), lp = Real(s_u[h][np]);
-                Nm.u[h] = im ? lm : Nm.u[h];
-                Np.u[h] = ip ? lp : Np.u[h];
-            }
-            const double qm = s_p64[nm], qp = s_p64[np];
-            Nm.p64 = im ? qm : Nm.p64;
-            Np.p64 = ip ? qp : Np.p64;
+        for (int h = 0; h < 5; ++h) {
+            const Real lm = Real(s_u[h][nm]), lp = Real(s_u[h][np]);
+            Nm.u[h] = im ? lm : Nm.u[h];
+            Np.u[h] = ip ? lp : Np.u[h];
         }
+        const double qm = s_p64[nm], qp = s_p64[np];
+        Nm.p64 = im ? qm : Nm.p64;
+        Np.p64 = ip ? qp : Np.p64;
     }
     make_state<D, false>(g, S0);
     make_state<D, false>(g, S1);
@@ -204,7 +202,7 @@ __device__ __forceinline__ void surface_pass(const StageArgs<M, Real>& a, long l
                                              const FaceNodes& fn) {
     const int tid = threadIdx.x;
     Real fm[5], fp[5], jac;
-    surface_fluxes<D, M, BE, SURF, true, Real, TU>(a, tid, e0, s_u, s_p64, geo, fn.m[D], fn.p[D], fm, fp, jac);
+    surface_fluxes<D, M, BE, SURF, Real, TU>(a, tid, e0, s_u, s_p64, geo, fn.m[D], fn.p[D], fm, fp, jac);
     surface_add<D, M, BE, Real>(a, tid, s_acc, fm, fp, jac);
 }
 

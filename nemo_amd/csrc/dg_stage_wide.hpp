@@ -149,7 +149,7 @@ __device__ __forceinline__ void stage_block_wide(const StageArgs<M, Real>& a, co
             geo.nbr[2 * D + 1] = int32_t(ep);
             geo.dx[D] = dx;
             Real jac;
-            surface_fluxes<D, M, BE, SURF, true, Real, TU>(a, ln, e0, s_u, s_p64, geo, um, up, fm, fp, jac);
+            surface_fluxes<D, M, BE, SURF, Real, TU>(a, ln, e0, s_u, s_p64, geo, um, up, fm, fp, jac);
             // the volume pass reads its nodes anew, as in stage_kernel: shared
             // with the face solves, its expressions would be contracted into
             // other FMAs (other last bits) and hold more registers
