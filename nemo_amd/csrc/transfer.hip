@@ -63,27 +63,42 @@ hipError_t launch_layout(hipStream_t stream, const double* src, double* dst, lon
 // Pinned staging of the copies over the host link.  A copy to or from
 // pageable memory runs at 10 GB/s into fresh pages (one thread of the runtime
 // copies and takes the page faults); four threads that each pipeline their
-// own two pinned chunks reach 43 GB/s both ways (two threads 26, eight 45;
-// 671 MB, fresh pages).  At 1.3 MB the plain copy takes 0.09 ms against 0.21
-// ms, at 13 MB 1.3 against 0.53, so the line is at 4 MB.  Chunks of 2 MB for
-// long transfers (39 GB/s with 1 MB); shorter transfers take smaller chunks,
-// so that all threads have several, and touch less of the pinned memory.
+// own two pinned chunks reach 45 to 51 GB/s both ways (671 MB).  ms per
+// transfer, plain copy -> staged:
+//   download into fresh pages    6 MB 0.82 -> 0.39, 13 MB 1.6 -> 0.65, 26 MB 2.7 -> 0.93, 49 MB 5.0 -> 1.5
+//   into pages touched before    6 MB 0.33 -> 0.22, 13 MB 0.75 -> 0.37, 26 MB 1.4 -> 0.60, 49 MB 4.7 -> 1.0
+//   upload                       6 MB 0.25 -> 0.26, 13 MB 0.49 -> 0.43, 20 MB 0.74 -> 0.58, 26 MB 0.95 -> 0.69
+// and at 1.3 MB a download 0.09 -> 0.21: so downloads are staged from 4 MB on,
+// uploads, whose pages have always been touched, from 8 MB on.  A chunk costs a
+// gap of 8 us on the link: 2 MB (upload of 671 MB on one stream 21.5 ms with
+// 1 MB, 16.8 with 2); short downloads take smaller ones, so that all threads
+// have a share of the page faults.
+//
+// Half of the threads copy on the caller's stream, half on a second one, which
+// fills the gaps (16.8 -> 13.0 ms).  More streams gain nothing, and the first
+// copies on each set up a hardware queue: with one for every thread the first
+// transfers of a process took 28 to 35 ms longer, with two 13 to 20.
 //
 // The calling thread and three helpers claim chunks one by one.  The caller
 // waits only for helpers that have claimed one, so a helper that the host's
 // scheduler keeps back (all cores busy, for instance with the spinning
 // threads of an OpenMP program) costs nothing: with threads of fixed shares,
 // started for each call, 40 downloads of 9 MB on average between such sections
-// took 38 ms longer.
+// took 38 ms longer.  A helper that loses its core after it has claimed one is
+// waited for: right after such a section a download of 6 MB takes 0.6 ms (plain
+// copy 0.4), of 13 MB 0.7 (0.8), of 49 MB 2.8 (5.6).
 constexpr int NT = 4, NBUF = 2 * NT;
-constexpr size_t CHUNK = size_t(2) << 20, MIN_BYTES = size_t(4) << 20;
+constexpr size_t MB = size_t(1) << 20, CHUNK = 2 * MB;
+constexpr size_t MIN_DOWNLOAD = 4 * MB, MIN_UPLOAD = 8 * MB;
 
-size_t chunk_for(size_t bytes) {
-    return bytes < (size_t(32) << 20) ? CHUNK / 4 : (bytes < (size_t(128) << 20) ? CHUNK / 2 : CHUNK);
+size_t chunk_for(size_t bytes, bool to_host) {
+    return !to_host || bytes >= 16 * MB ? CHUNK : (bytes < 8 * MB ? CHUNK / 4 : CHUNK / 2);
 }
 
-// One transfer: chunks [0, nc) of `chunk` bytes between dev and host.
+// One transfer: chunks [0, nc) of `chunk` bytes between dev and host; thread k
+// copies on stream[k & 1].
 struct Job {
+    hipStream_t stream[2];
     char* dev;
     char* host;
     size_t bytes, chunk, nc;
@@ -99,8 +114,8 @@ public:
         Staging* s = new (std::nothrow) Staging();
         if (!s) return nullptr;
         bool ok = hipHostMalloc(reinterpret_cast<void**>(&s->pinned_), NBUF * CHUNK, hipHostMallocDefault) == hipSuccess;
-        for (auto& x : s->stream_) ok = ok && hipStreamCreateWithFlags(&x, hipStreamNonBlocking) == hipSuccess;
         for (auto& x : s->done_) ok = ok && hipEventCreateWithFlags(&x, hipEventDisableTiming) == hipSuccess;
+        ok = ok && hipStreamCreateWithFlags(&s->second_, hipStreamNonBlocking) == hipSuccess;
         ok = ok && hipEventCreateWithFlags(&s->start_, hipEventDisableTiming) == hipSuccess;
         if (!ok) {
             (void)hipGetLastError();
@@ -124,8 +139,7 @@ public:
         wake_.notify_all();
         for (auto& t : helper_)
             if (t.joinable()) t.join();
-        for (auto& x : stream_)
-            if (x) (void)hipStreamDestroy(x);
+        if (second_) (void)hipStreamDestroy(second_);
         for (auto& x : done_)
             if (x) (void)hipEventDestroy(x);
         if (start_) (void)hipEventDestroy(start_);
@@ -135,9 +149,10 @@ public:
     // The whole transfer, after the work already on `stream`; one at a time.
     hipError_t copy(hipStream_t stream, Job& job) {
         hipError_t rc = hipEventRecord(start_, stream);
-        for (auto& x : stream_)
-            if (rc == hipSuccess) rc = hipStreamWaitEvent(x, start_, 0);
+        if (rc == hipSuccess) rc = hipStreamWaitEvent(second_, start_, 0);
         if (rc != hipSuccess) return rc;
+        job.stream[0] = stream;
+        job.stream[1] = second_;
         {
             std::lock_guard<std::mutex> l(mu_);
             job_ = &job;
@@ -174,23 +189,20 @@ private:
     void work(int k, Job& j) {
         char* const buf[2] = {pinned_ + size_t(2 * k) * CHUNK, pinned_ + size_t(2 * k + 1) * CHUNK};
         hipEvent_t* const done = done_ + 2 * k;
+        const hipStream_t stream = j.stream[k & 1];
         hipError_t e = hipSuccess;
         auto len = [&](size_t c) { return std::min(j.chunk, j.bytes - c * j.chunk); };
         auto claim = [&] { return j.next.fetch_add(1); };
         auto link = [&](size_t c, int b) {
             char* const d = j.dev + c * j.chunk;
-            e = j.to_host ? hipMemcpyAsync(buf[b], d, len(c), hipMemcpyDeviceToHost, stream_[k])
-                          : hipMemcpyAsync(d, buf[b], len(c), hipMemcpyHostToDevice, stream_[k]);
-            if (e == hipSuccess) e = hipEventRecord(done[b], stream_[k]);
+            e = j.to_host ? hipMemcpyAsync(buf[b], d, len(c), hipMemcpyDeviceToHost, stream)
+                          : hipMemcpyAsync(d, buf[b], len(c), hipMemcpyHostToDevice, stream);
+            if (e == hipSuccess) e = hipEventRecord(done[b], stream);
         };
-        bool any = false;
         int b = 0;
         if (j.to_host) {
             size_t c = claim();
-            if (c < j.nc) {
-                any = true;
-                link(c, 0);
-            }
+            if (c < j.nc) link(c, 0);
             while (c < j.nc && e == hipSuccess) {
                 const size_t ahead = claim();
                 if (ahead < j.nc) link(ahead, b ^ 1);
@@ -202,27 +214,24 @@ private:
         } else {
             int used = 0;
             for (size_t c = claim(); c < j.nc && e == hipSuccess; c = claim(), b ^= 1) {
-                any = true;
                 if (used >= 2) e = hipEventSynchronize(done[b]);
                 if (e != hipSuccess) break;
                 std::memcpy(buf[b], j.host + c * j.chunk, len(c));
                 link(c, b);
                 ++used;
             }
-        }
-        // nothing is left in flight, also after an error
-        if (any) {
-            const hipError_t last = hipStreamSynchronize(stream_[k]);
-            if (e == hipSuccess) e = last;
+            // (the last copy of either buffer; downloads have waited for theirs)
+            for (int q = 0; q < 2 && q < used && e == hipSuccess; ++q) e = hipEventSynchronize(done[q]);
         }
         if (e != hipSuccess) {
+            (void)hipStreamSynchronize(stream);  // nothing is left in flight
             j.err.store(int(e));
             j.next.store(j.nc);
         }
     }
 
     char* pinned_ = nullptr;  // NBUF chunks of CHUNK bytes
-    hipStream_t stream_[NT] = {};
+    hipStream_t second_ = nullptr;
     hipEvent_t done_[NBUF] = {};
     hipEvent_t start_ = nullptr;
     std::thread helper_[NT];
@@ -258,7 +267,7 @@ bool staged_copy(hipStream_t stream, double* dev, double* host, size_t bytes, bo
     job.dev = reinterpret_cast<char*>(dev);
     job.host = reinterpret_cast<char*>(host);
     job.bytes = bytes;
-    job.chunk = chunk_for(bytes);
+    job.chunk = chunk_for(bytes, to_host);
     job.nc = (bytes + job.chunk - 1) / job.chunk;
     job.to_host = to_host;
     *err = staging[device]->copy(stream, job);
@@ -323,7 +332,7 @@ hipError_t state_to_host(hipStream_t stream, const double* dev, long long stride
     const size_t bytes = size_t(ne) * V * M3 * sizeof(double);
     hipError_t e = launch_layout<true>(stream, dev, scratch, stride, off, ne, V, M3);
     if (e != hipSuccess) return e;
-    if (bytes >= MIN_BYTES && staged_copy(stream, scratch, host, bytes, true, &e)) return e;
+    if (bytes >= MIN_DOWNLOAD && staged_copy(stream, scratch, host, bytes, true, &e)) return e;
     e = hipMemcpyAsync(host, scratch, bytes, hipMemcpyDeviceToHost, stream);
     return e != hipSuccess ? e : hipStreamSynchronize(stream);
 }
@@ -332,7 +341,7 @@ hipError_t state_to_device(hipStream_t stream, const double* host, double* scrat
                            long long off, long long ne, int V, int M3) {
     const size_t bytes = size_t(ne) * V * M3 * sizeof(double);
     hipError_t e = hipSuccess;
-    if (bytes < MIN_BYTES || !staged_copy(stream, scratch, const_cast<double*>(host), bytes, false, &e)) {
+    if (bytes < MIN_UPLOAD || !staged_copy(stream, scratch, const_cast<double*>(host), bytes, false, &e)) {
         e = hipMemcpyAsync(scratch, host, bytes, hipMemcpyHostToDevice, stream);
         // the host array is the caller's again on return
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
