@@ -7,8 +7,8 @@
 // elements (own neighbour, constant state, element size 1e30, so they stay
 // constant and never set a time step), so that a block of BE elements
 // belongs to one run; a per-block run table gives the block its run's dt.
-// Per RK stage one persistent launch per group walks all blocks of all its
-// runs; the CFL partials of each block are reduced per run.  A pair of time
+// Per RK stage one launch covers the blocks of all groups, or one launch per
+// group its own; the CFL partials of each block are reduced per run.  A pair of time
 // steps (ten stage flips, so the ping-pong buffers return to their start) is
 // captured as a HIP graph and replayed.
 #include <hip/hip_runtime.h>
@@ -158,7 +158,7 @@ void launch_group_stage(Batch* b, hipStream_t stream, Group& gr, int stage, bool
     if (b->grid_per_cu == 0 && wide_form<M, Real>(b->cfg, b->form, gr.nblocks)) {
         // few blocks: each on four wavefronts, with the same bits (4 runs of 5
         // to 9 elements a side, FP64: 102 -> 59 us per stage of all degrees; 8
-        // runs of 6 to 12, FP32: 88 -> 60)
+        // runs of 6 to 12, FP32: 88 -> 60; before the groups had streams)
         hipLaunchKernelGGL((nemo::stage_kernel_wide<nemo::EQ_EULER, M, BE, nemo::VOL_EC, nemo::SURF_HLLC, Real>),
                            dim3(unsigned(gr.nblocks)), dim3(nemo::WIDE_NT), 0, stream, a);
         return;

@@ -1156,7 +1156,7 @@ __device__ __forceinline__ void block_cfl_nodes(const Phys64& P, const double* _
 }
 
 // Up to this many blocks the one that finishes last reduces the partials of
-// all (eight loads per thread, all in flight at once), and the reduction needs
+// all (eight per thread, whose 24 loads are all in flight at once), and the reduction needs
 // no launch of its own (7 us and a gap, against 11 us for a whole stage of 8^3
 // elements; more partials would be read in several rounds by one CU).
 constexpr int CFL_FUSE = 2048;
@@ -1202,8 +1202,10 @@ __device__ __forceinline__ void cfl_last_block(const double* part, int grid, con
 
 // Standalone CFL reduction of a state in HBM (first step, calc_timestep): the
 // same per-block partials as the stage kernels' epilogues, a node per thread.
-// Bound by the read of the state (64^3, 671 MB: 331 us with one wavefront per
-// block and the block staged in LDS, 252 us now).
+// Bound by the LDS maxima: the 64 nodes of an element meet at four addresses,
+// and wavefronts wait to issue LDS operations for 47 % of their cycles (counters
+// on 64^3, 671 MB: 331 us with one wavefront per block and the block staged in
+// LDS, 250 us now, 2.7 TB/s; a copy of the state runs at 5.4).
 template <int EQ, int M, int BE>
 __global__ __launch_bounds__(CFL_NT) void cfl_kernel(const double* __restrict__ u, const double* __restrict__ delta,
                                                      long long nelem, Phys64 P, double* part, CflFinal fin) {

@@ -127,11 +127,11 @@ __device__ __forceinline__ void mlp_forward_wave(const float* __restrict__ P, co
 // unit) are consecutive.  The weights stay in registers over all tiles of a
 // workgroup; activations and deltas change hands through LDS.
 //
-// What bounds them: the chain of layers of one tile (about 100 matrix
-// instructions a wavefront and five barriers); the arithmetic of 4096 samples
-// is 2 us at the FP32 matrix rate.  One sample at a time per wavefront, with
-// the other units' activations by v_readlane, took 98 us for the gradient of
-// 4096 samples and 74 us for the outputs of 100 000.
+// What bounds them: the chain of layers of one tile (gradient: about 100 matrix
+// instructions a wavefront and seven barriers; outputs: 33 and four); the
+// arithmetic of 4096 samples is 2 us at the FP32 matrix rate.  One sample at a
+// time per wavefront, with the other units' activations by v_readlane, took
+// 98 us for the gradient of 4096 samples and 74 us for the outputs of 100 000.
 constexpr int MLP_TILE = 16;   // samples of a tile
 constexpr int MLP_NT = 256;    // four wavefronts
 constexpr int MLP_LD = 68;     // row of an LDS tile: 16-byte aligned, rows four banks apart

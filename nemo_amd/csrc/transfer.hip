@@ -21,7 +21,7 @@ namespace {
 // the other, so both sides coalesce.  It takes the place of a second host
 // array as large as the state and a row-by-row memcpy on one host thread: a
 // download of 262 144 elements of 5 x 64 (671 MB) took 205 ms with them and
-// takes 16 to 22 ms now, with the staging below.
+// takes 15 to 17 ms now, with the staging below.
 template <int V, int M3, bool TO_HOST>
 __global__ __launch_bounds__(256) void layout_kernel(const double* __restrict__ src, double* __restrict__ dst,
                                                      long long stride, long long off, long long ne) {
