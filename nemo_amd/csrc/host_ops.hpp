@@ -17,8 +17,11 @@ namespace nemo_host {
 // Last error message of the calling thread (nemo_gpu_error_message).
 std::string& last_error();
 
+// The error is reported here: the runtime's record of it is cleared, so that
+// the check behind a later launch of the thread does not find it.
 inline int fail(int code, const std::string& msg) {
     last_error() = msg;
+    if (code == NEMO_ERR_HIP) (void)hipGetLastError();
     return code;
 }
 

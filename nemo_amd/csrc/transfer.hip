@@ -39,17 +39,19 @@ __global__ __launch_bounds__(256) void layout_kernel(const double* __restrict__ 
     }
 }
 
+// Returns the launch's own error: the thread's last error may be an earlier
+// call's (a failed allocation, another library's), which is no reason to refuse
+// a transfer.
 template <bool TO_HOST>
 hipError_t launch_layout(hipStream_t stream, const double* src, double* dst, long long stride, long long off,
                          long long ne, int V, int M3) {
     const long long n = ne * V * M3;
     const dim3 grid{unsigned(std::min<long long>((n + 255) / 256, 1 << 20))}, block{256};
-#define NEMO_LAYOUT(V_, M3_)                                                                                \
-    if (V == V_ && M3 == M3_) {                                                                             \
-        hipLaunchKernelGGL((layout_kernel<V_, M3_, TO_HOST>), grid, block, 0, stream, src, dst, stride, off, \
-                           ne);                                                                             \
-        return hipGetLastError();                                                                           \
-    }
+    void* args[] = {&src, &dst, &stride, &off, &ne};
+#define NEMO_LAYOUT(V_, M3_)   \
+    if (V == V_ && M3 == M3_)  \
+        return hipLaunchKernel(reinterpret_cast<const void*>(&layout_kernel<V_, M3_, TO_HOST>), grid, block, args, 0, \
+                               stream);
     NEMO_LAYOUT(5, 27)
     NEMO_LAYOUT(5, 64)
     NEMO_LAYOUT(5, 125)
